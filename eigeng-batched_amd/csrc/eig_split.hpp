@@ -63,12 +63,14 @@ __device__ __forceinline__ int sw_ilo(int code) { return (code >> 20) & 1023; }
 // LIST (NB = 64 and 128): the uneven-batch form (u), one workgroup per slot of
 // the chunk, its own order n from nv, packed input at a + aoff, Q slot nmx^2
 // (leading dimension n), d / e at rows i / nmx + i of de.
+// only (may be null): just the matrices flagged ST_OVERFLOW there.
 template <typename T, int NB, bool LIST = false>
 __global__ __launch_bounds__(64 * GroupShape<NB>::NW) void eig_tri_kernel(int L, int nm, int n,
                                                                         const T *__restrict__ a,
                                                                         T *__restrict__ qws,
                                                                         T *__restrict__ de, int ld,
-                                                                        UvSplitArgs u = UvSplitArgs{})
+                                                                        UvSplitArgs u = UvSplitArgs{},
+                                                                        const int *__restrict__ only = nullptr)
 {
   // NB <= 64: groups of NB lanes; NB = 128: two waves per matrix, row k of
   // the matrix in lane k % 64 of wave k / 64
@@ -91,6 +93,7 @@ __global__ __launch_bounds__(64 * GroupShape<NB>::NW) void eig_tri_kernel(int L,
     Q = qws + (size_t)mat * u.nmx * u.nmx;
   } else {
     if (mat >= L) return;                            // the whole group (G = 1 when NW > 1)
+    if (only && only[mat] != ST_OVERFLOW) return;
     eoff = n;
     A = a + (size_t)mat * (size_t)nm * (size_t)n;
     Q = qws + (size_t)mat * (size_t)n * (size_t)n;

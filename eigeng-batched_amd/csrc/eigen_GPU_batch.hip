@@ -18,6 +18,7 @@
 #include "eig_uneven.hpp"
 #include "eig_split_large.hpp"
 #include "eig_tri_reg.hpp"
+#include "eig_dc.hpp"
 #include "eig_check.hpp"
 #include "eig_symdmt.hpp"
 #include "eig_gemm.hpp"
@@ -66,7 +67,13 @@ constexpr int FLAG_UNSORTED = 0x40000000;
 // FP64 refinement on MFMA (eig_refine.hpp) with the plain FP64 solver as the
 // fallback for matrices the refinement does not accept
 constexpr int SOLVER_MIXED = 3;
-// with SOLVER_MIXED, 64 < n <= 256: the FP32 stage takes the large-order split
+// IMTQL2: the divide and conquer path (eig_dc.hpp), also where the rule of
+// use_dc would not take it (the autotuner's name for that path)
+constexpr int FLAG_DC = 0x8000000;
+// internal (workspace sizes): the path that a call takes without divide and
+// conquer (bits 28-29 belong to SOLVER_MIXED and mean nothing to IMTQL2)
+constexpr int FLAG_ROUTE_QL = 0x10000000;
+// with SOLVER_MIXED, 64 < n <= 256 (the same bit): the FP32 stage takes the large-order split
 // path with the back-transformation as blocked reflectors on the matrix cores
 // (FP16-split products, eig_wy.hpp) instead of forming Q on the vector units
 constexpr int FLAG_MIXED_WY16 = 0x8000000;
@@ -182,6 +189,48 @@ bool use_split128(int L, int n, int tbytes, int solver)
   return L >= SPLIT_MIN_L;
 }
 
+// Divide and conquer (eig_dc.hpp): the sorted IMTQL2 interface without a path
+// choice of the caller's (chunk and phase bits aside), 8 <= n <= 64.  Measured on
+// one MI355X, random symmetric matrices, against the better of the fused and the
+// split path (us, that / divide and conquer): L = 64: n = 8 42 / 23 (FP32), 50 / 29
+// (FP64); n = 16 104 / 28, 132 / 40; n = 32 277 / 60, 363 / 75; n = 64 819 / 157,
+// 1094 / 188.  L = 2048: n = 8 44 / 25, 54 / 37; n = 16 110 / 38, 145 / 56; n = 32
+// 300 / 85, 399 / 121; n = 64 912 / 263, 1393 / 452.  On large batches the QL
+// recurrence's latency is shared by more matrices, and orders that fill their
+// padded tiles badly lose: L = 16384: n = 8 52 / 67, 78 / 142; n = 9 80 / 86,
+// 101 / 175; n = 12 103 / 90, 146 / 189; n = 20 258 / 213, 385 / 443; n = 33
+// 784 / 667, 1372 / 1489; n = 40 990 / 764, 1802 / 1690; n = 64 1915 / 1364,
+// 3742 / 3190; those keep the QL paths from about where the two lines cross.
+constexpr int DC_MIN_N = 8;
+int dc_max_l(int n, int tbytes)
+{
+  if (n <= 8) return 4096;
+  if (tbytes == 4) return n <= 10 ? 12288 : 0x7fffffff;
+  if (n <= 16) return 6144;
+  return (n <= 23) ? 8192 : (n >= 33 && n <= 37) ? 12288 : 0x7fffffff;
+}
+// FLAG_SPLIT asks for the path in separate kernels: on batches that take it by
+// themselves that is this one, smaller ones get the QL recurrence.
+bool use_dc(int L, int n, int tbytes, int solver)
+{
+  const int flags = solver & ~0xff & ~(3 << CHUNK_SHIFT) & ~FLAG_PH_ALL;
+  if ((solver & 0xff) != SOLVER_IMTQL2 || (flags & ~(FLAG_DC | FLAG_SPLIT)) || n > 64) return false;
+  if (flags & FLAG_DC) return true;
+  return n >= DC_MIN_N && L <= dc_max_l(n, tbytes) && (!(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L);
+}
+
+// Workspace of the divide and conquer path, n <= 64, for a chunk of lc matrices:
+// Q, d / e.
+struct DcLayout {
+  size_t q, de, total;
+  DcLayout(int lc, int n, int tb)
+  {
+    q = 0;
+    de = q + al256((size_t)lc * n * n * tb);
+    total = de + al256((size_t)2 * n * lc * tb);
+  }
+};
+
 int global_grid(int L) { return L < 1024 ? L : 1024; }
 
 // Workspace: the register kernels keep everything in registers and LDS (a
@@ -245,7 +294,14 @@ bool mixed_wy(int n, int solver) { return (solver & FLAG_MIXED_WY16) && n > 64; 
 
 size_t workspace_bytes(int L, int nm, int n, int m, int tbytes, int solver)
 {
-  (void)nm; (void)m;
+  if (use_dc(L, n, tbytes, solver)) {
+    // at least what the path without it asks for, so that a tuned choice of
+    // that path fits in a workspace of the size the query reports
+    const size_t other = workspace_bytes(L, nm, n, m, tbytes, (solver & ~FLAG_DC) | FLAG_ROUTE_QL);
+    const size_t own = WS_HEAD + DcLayout(L < lchunk(solver) ? L : lchunk(solver), n, tbytes).total;
+    return own > other ? own : other;
+  }
+  solver &= ~FLAG_ROUTE_QL;
   if ((solver & 0xff) == SOLVER_MIXED) {
     if (tbytes != 8 || n > 256) return 0;
     return WS_HEAD + MixedLayout(L, n, mixed_wy(n, solver), solver & (3 << CHUNK_SHIFT)).total;
@@ -311,6 +367,55 @@ hipError_t launch_split(int L, int nm, int n, T *a, T *w, int *info, int solver,
       hipLaunchKernelGGL((eig_wave_kernel<T, NB>), dim3(gb), dim3(64 * NW), 0, s, cur, nm, n, ac, wc, ic,
                          kop, (const int *)st);
     }
+  }
+  return hipGetLastError();
+}
+
+// Divide and conquer path for n <= 64 on one chunk: q, de (ld rows apart) as in
+// DcLayout.  Phases: tridiagonalisation with Q; the second one nothing; merges and
+// store.  nanfail, only: see eig_dc_kernel.
+template <typename T, int NB, int NBT, int NLR>
+void launch_dc_chunk(int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, int nanfail, T *q, T *de, int ld,
+                     const int *only, hipStream_t s)
+{
+  constexpr int G = GroupShape<NBT>::G;
+  if (ph & FLAG_PH_TRI)
+    hipLaunchKernelGGL((eig_tri_kernel<T, NBT>), dim3((unsigned)((cur + G - 1) / G)), dim3(64), 0, s, cur, nm, n, a, q,
+                       de, ld, UvSplitArgs{}, only);
+  if (ph & FLAG_PH_APPLY)
+    hipLaunchKernelGGL((eig_dc_kernel<T, NB, NLR, false>), dim3((unsigned)cur), dim3(NB * NLR), 0, s, cur, nm, n, a,
+                       (const T *)q, (const T *)de, ld, w, info, kop, nanfail, 1, (T *)nullptr, only);
+}
+template <typename T>
+void dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, T *q, T *de, int ld,
+              const int *only, hipStream_t s)
+{
+  const int nanfail = L < split_min_l(n, (int)sizeof(T)) ? 1 : 0;
+#define DC(NB, NBT, NLR) launch_dc_chunk<T, NB, NBT, NLR>(cur, nm, n, a, w, info, ph, kop, nanfail, q, de, ld, only, s)
+  if (n <= 8) DC(16, 8, 4);
+  else if (n <= 16) DC(16, 16, 4);
+  // one wave a matrix does fewer instructions, two have the shorter chain
+  // (FP32 n = 32, L = 16384: 147 / 190 us; n = 20, L = 16: 24 / 20 us)
+  else if (n <= 32 && L < 512) DC(32, 32, 4);
+  else if (n <= 32) DC(32, 32, 2);
+  else if (n <= 48) DC(48, 64, 4);
+  else DC(64, 64, 4);
+#undef DC
+}
+
+template <typename T>
+hipError_t run_dc(int L, int nm, int n, T *a, T *w, int *info, int solver, int kop, void *wk, hipStream_t s)
+{
+  const int lc = L < lchunk(solver) ? L : lchunk(solver);
+  const DcLayout lay(lc, n, (int)sizeof(T));
+  char *base = (char *)wk + WS_HEAD;
+  T *q = (T *)(base + lay.q), *de = (T *)(base + lay.de);
+  const int ph = (solver & FLAG_PH_ALL) ? (solver & FLAG_PH_ALL) : FLAG_PH_ALL;
+  if (ph != FLAG_PH_ALL && L > lc) return hipErrorInvalidValue;
+  for (long long c0 = 0; c0 < L; c0 += lc) {
+    const int cur = (int)((L - c0) < lc ? (L - c0) : lc);
+    dc_chunk<T>(L, cur, nm, n, a + (size_t)c0 * nm * n, w + (size_t)c0 * n, info ? info + c0 : nullptr, ph, kop, q, de,
+                lc, nullptr, s);
   }
   return hipGetLastError();
 }
@@ -825,6 +930,7 @@ hipError_t run(int L, int nm, int n, int m, T *a, T *w, void *wk, hipStream_t s,
   if (wk == nullptr) return hipErrorInvalidValue;
   // kernel options: solver, order of the output, eigenvector columns not stored
   const int kop = kopt_make(base, (solver & FLAG_UNSORTED) != 0, n - m);
+  if (use_dc(L, n, (int)sizeof(T), solver)) return run_dc<T>(L, nm, n, a, w, info, solver, kop, wk, s);
   if ((solver & FLAG_PH_ALL) && !use_split(L, n, (int)sizeof(T), solver) && !use_split_large(L, n, (int)sizeof(T), solver) &&
       !use_split128(L, n, (int)sizeof(T), solver))
     return hipErrorInvalidValue;
@@ -868,6 +974,7 @@ std::vector<int> tune_candidates(int L, int n, int tb, int solver)
   if (use_wave_kernel(n, tb)) {
     c.push_back(FLAG_FUSED);
     if (n <= 64) {
+      if (base == SOLVER_IMTQL2) c.push_back(FLAG_DC);
       c.push_back(FLAG_SPLIT);
       c.push_back(FLAG_SPLIT | FLAG_QL_LDS);
       c.push_back(FLAG_SPLIT | (1 << CHUNK_SHIFT));
@@ -1295,7 +1402,11 @@ hipError_t run_warm(int L, int nm, int n, int m, T *a, const T *q0, T *w, void *
     if ((err = gemm_launch(kind, g, s)) != hipSuccess) return err;
     hipLaunchKernelGGL((eig_warm_store_kernel<T>), dim3((unsigned)(cur < 16384 ? cur : 16384)), dim3(256), 0, s, cur,
                        nm, n, m, (const T *)v, (const int *)ji, st, ac, ic);
-    if (n <= 8) launch_wave_only<T, 8>(cur, nm, n, ac, wc, ic, kop, st, s);
+    // the matrices left over: the path a plain call of this batch takes (small
+    // batches' when that is a QL one), in the regions that are free by now
+    if (use_dc(L, n, tb, SOLVER_IMTQL2))
+      dc_chunk<T>(L, cur, nm, n, ac, wc, ic, FLAG_PH_ALL, kop, ab, q, cur, st, s);
+    else if (n <= 8) launch_wave_only<T, 8>(cur, nm, n, ac, wc, ic, kop, st, s);
     else if (n <= 16) launch_wave_only<T, 16>(cur, nm, n, ac, wc, ic, kop, st, s);
     else if (n <= 32) launch_wave_only<T, 32>(cur, nm, n, ac, wc, ic, kop, st, s);
     else launch_wave_only<T, 64>(cur, nm, n, ac, wc, ic, kop, st, s);
@@ -1609,7 +1720,9 @@ hipError_t launch_params(int L, int n, int tb, int solver, int *p)
     p[3] = threads;
     p[1] = (nmat + g - 1) / g;
   };
-  if (tb == 4 && use_split128(L, n, tb, solver)) {
+  if (use_dc(L, n, tb, solver)) {
+    grp(nb_of(n), L < lchunk(solver) ? L : lchunk(solver), 64);
+  } else if (tb == 4 && use_split128(L, n, tb, solver)) {
     grp(128, L < lchunk(solver) ? L : lchunk(solver), 128);
   } else if (use_split(L, n, tb, solver)) {
     grp(nb_of(n), L < lchunk(solver) ? L : lchunk(solver), 64);

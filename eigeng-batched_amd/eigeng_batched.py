@@ -38,11 +38,13 @@ FLAG_TRI_FULL = 0x4000000
 TRI_CFG_SHIFT = 24
 FLAG_TRI_WS = 1 << TRI_CFG_SHIFT
 FLAG_REG128 = 0x8000
+# the divide and conquer tridiagonal solver (IMTQL2; the default, csrc/eig_dc.hpp)
+FLAG_DC = 0x8000000
 # eigenpairs in the QL / Jacobi order instead of ascending (the reference's DO_SORT 0)
 FLAG_UNSORTED = 0x40000000
 # bits 18-19: the split paths' batch chunk divided by 2, 4 or 8 (smaller workspace, longer call)
 CHUNK_SHIFT = 18
-PATHS = {"auto": 0, "fused": FLAG_FUSED, "split": FLAG_SPLIT, "split-fallback": FLAG_SPLIT | FLAG_TINYLOG,
+PATHS = {"auto": 0, "dc": FLAG_DC, "fused": FLAG_FUSED, "split": FLAG_SPLIT, "split-fallback": FLAG_SPLIT | FLAG_TINYLOG,
          "split-lds": FLAG_SPLIT | FLAG_QL_LDS, "split-full": FLAG_SPLIT | FLAG_TRI_FULL,
          "split-ws": FLAG_SPLIT | FLAG_TRI_WS,
          "split-reg128": FLAG_REG128, "split-reg128-fallback": FLAG_REG128 | FLAG_TINYLOG}
@@ -182,8 +184,10 @@ def eigen_batch(a, w=None, m: int | None = None, solver: int = IMTQL2, info=None
     ``a[k, j, :n]``), ``w`` (L, n) ascending eigenvalues, ``info`` (L,) int32
     per-matrix status (0 ok, l>0 QL did not converge) or None when abi=True.
     abi=True calls the reference-compatible eigen_GPU_batch_FP/_DP symbol.
-    path selects the n <= 64 implementation: "auto", "fused" (one kernel),
-    "split" (lane-per-matrix QL recurrence) or "split-fallback" (split with the
+    path selects the n <= 64 implementation: "auto", "fused" (one kernel), "dc"
+    (divide and conquer, what "auto" takes for most shapes), "split" (separate
+    kernels: divide and conquer from 2048 matrices on, below that the
+    lane-per-matrix QL recurrence) or "split-fallback" (split with the
     rotation log shrunk so that every matrix takes the overflow fallback) or
     "split-lds" (split with the QL recurrence's d, e kept in LDS rather than in
     registers) or, for 64 < n <= 256, "split-full" (split with the
