@@ -639,8 +639,8 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
 // workgroup per matrix.  X starts as Q^T, so the last merge leaves the
 // eigenvectors of A themselves.
 // BLK: a 64-column block of a larger matrix (nblk per matrix) with X starting from
-// the identity: the block's eigenvectors of T to zout (ld n, at (64 b, 64 b)) and
-// its eigenvalues to w.
+// the identity: the block's eigenvectors of T to z0 or z1 (bit b of zmask; ld n,
+// at (64 b, 64 b)) and its eigenvalues to w (NaN for a block that is not finite).
 // nanfail: what a matrix that is not finite gives: 1: info = 1 and a untouched,
 // 0: the diagonal and Q as they are (sorted by the reference's rule), info = 0
 // (the two outcomes of the QL paths, by batch size).
@@ -648,8 +648,8 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
 template <typename T, int NB, int NLR, bool BLK>
 __global__ __launch_bounds__(NB *NLR) __attribute__((amdgpu_waves_per_eu(DcTune<T, NB>::WAVES))) void eig_dc_kernel(
     int L, int nm, int n_all, T *__restrict__ a, const T *__restrict__ qws, const T *__restrict__ de, int ld,
-    T *__restrict__ w, int *__restrict__ info, int opts, int nanfail, int nblk, T *__restrict__ zout,
-    const int *__restrict__ only)
+    T *__restrict__ w, int *__restrict__ info, int opts, int nanfail, int nblk, T *__restrict__ z0,
+    T *__restrict__ z1, int zmask, const int *__restrict__ only)
 {
   typedef typename Mfma16<T>::v4 v4;
   typedef DcShape<NB, NLR> G;
@@ -817,7 +817,7 @@ __global__ __launch_bounds__(NB *NLR) __attribute__((amdgpu_waves_per_eu(DcTune<
 
   if (sub == 0 && lv) wout[i] = Sh.d[i] * isc;
   if (!BLK && info && tid == 0) info[mat] = 0;
-  T *__restrict__ O = BLK ? zout + (size_t)mat * n_all * n_all + (size_t)b0 * n_all + b0
+  T *__restrict__ O = BLK ? (((zmask >> (b0 / 64)) & 1) ? z1 : z0) + (size_t)mat * n_all * n_all + (size_t)b0 * n_all + b0
                           : a + (size_t)mat * (size_t)nm * (size_t)n;
   const int ldo = BLK ? n_all : nm, mcols = BLK ? n : n - kopt_mdrop(opts);
 #pragma unroll

@@ -61,6 +61,7 @@ struct GemmArgs {
   void *C; long long ldc, sc;
   double alpha, beta;
   int sym;                              // 0, or the width (in 64-wide tiles) of the symmetric blocks
+  const int *skip;                      // may be null: products b with skip[b] != 0 are left out
 };
 
 constexpr int GM_TILE = 64, GM_KC = 16, GM_THREADS = 256, GM_PAD = 4;
@@ -245,50 +246,27 @@ __device__ __forceinline__ long long gemm_xcd_remap(long long bid, long long tot
 // Each thread loads 4 elements of the 64 x 16 A chunk and 4 of the 16 x 64 B
 // chunk.  Non-transposed A (rows contiguous): thread t takes row t & 63 and k =
 // (t >> 6) + 4 i; transposed A (k contiguous): k = t & 15, row = (t >> 4) + 16 i.
-// B likewise with the roles of rows and k exchanged.
-// held to 128 registers (four waves per SIMD): with the second chunk buffer
-// the FP64 kind otherwise takes 136 and runs at three
+// B likewise with the roles of rows and k exchanged.  acc (and acc2 for GK_F16X3):
+// wave q's 32 x 32 quarter of the tile at (row0, col0) of op(A) op(B).
 template <int KIND>
-__global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void eig_gemm_kernel(GemmArgs g)
+struct alignas(16) GemmLds {
+  // two chunk buffers: the next chunk is stored while the current one is
+  // multiplied, with one barrier per chunk
+  typename GemmT<KIND>::L A[2][GM_KC][GM_TILE + GM_PAD];
+  typename GemmT<KIND>::L B[2][GM_KC][GM_TILE + GM_PAD];
+};
+template <int KIND>
+__device__ __forceinline__ void gemm_tile(int M, int N, int K, int transa, int transb,
+                                          const typename GemmT<KIND>::S *__restrict__ A, long long lda,
+                                          const typename GemmT<KIND>::S *__restrict__ B, long long ldb, int row0,
+                                          int col0, GemmLds<KIND> &Sm, typename GemmT<KIND>::v4 (&acc)[2][2],
+                                          typename GemmT<KIND>::v4 (&acc2)[2][2])
 {
   typedef GemmT<KIND> TT;
   typedef typename TT::S S;
   typedef typename TT::L Ls;
-  typedef typename TT::v4 v4;
-  // two chunk buffers: the next chunk is stored while the current one is
-  // multiplied, with one barrier per chunk
-  __shared__ Ls As[2][GM_KC][GM_TILE + GM_PAD];
-  __shared__ Ls Bs[2][GM_KC][GM_TILE + GM_PAD];
-
-  const int tm = (g.M + GM_TILE - 1) / GM_TILE, tn = (g.N + GM_TILE - 1) / GM_TILE;
-  long long tiles;
-  int symw = g.sym;
-  if (symw > 0) {
-    // tn = nblk * symw tiles in blocks of symw x symw (tm == symw)
-    tiles = (long long)(tn / symw) * (symw * (symw + 1) / 2);
-  } else {
-    tiles = (long long)tm * tn;
-  }
-  const long long total = tiles * g.batch;
-  const long long lid = gemm_xcd_remap(blockIdx.x, total);
-  if (lid >= total) return;
-  const long long b = lid / tiles;
-  int t = (int)(lid - b * tiles), ti, tj;
-  if (symw > 0) {
-    const int per = symw * (symw + 1) / 2;
-    const int blk = t / per;
-    int r = t - blk * per, J = 0;
-    while ((J + 1) * (J + 2) / 2 <= r) ++J;
-    ti = r - J * (J + 1) / 2;
-    tj = blk * symw + J;
-  } else {
-    ti = t % tm;
-    tj = t / tm;
-  }
-  const int row0 = ti * GM_TILE, col0 = tj * GM_TILE;
-  const S *__restrict__ A = (const S *)g.A + b * g.sa;
-  const S *__restrict__ B = (const S *)g.B + b * g.sb;
-
+  Ls (*As)[GM_KC][GM_TILE + GM_PAD] = Sm.A;
+  Ls (*Bs)[GM_KC][GM_TILE + GM_PAD] = Sm.B;
   const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
   const int m = lane & 15, gg = lane >> 4;
   const int wr = (q & 1) * 32, wc = (q >> 1) * 32;
@@ -297,22 +275,22 @@ __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   int ar[4], ak[4], bk[4], bc[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (!g.transa) { ar[i] = tid & 63; ak[i] = (tid >> 6) + 4 * i; }
+    if (!transa) { ar[i] = tid & 63; ak[i] = (tid >> 6) + 4 * i; }
     else { ak[i] = tid & 15; ar[i] = (tid >> 4) + 16 * i; }
-    if (!g.transb) { bk[i] = tid & 15; bc[i] = (tid >> 4) + 16 * i; }
+    if (!transb) { bk[i] = tid & 15; bc[i] = (tid >> 4) + 16 * i; }
     else { bc[i] = tid & 63; bk[i] = (tid >> 6) + 4 * i; }
   }
   // every load is issued, from indices clamped into the operand, and
   // out-of-range elements become zero when the chunk is stored to LDS: with no
   // branch or select after them the loads of the next chunks stay in flight
   // across this chunk's products
-  const long long lsa_r = g.transa ? g.lda : 1, lsa_k = g.transa ? 1 : g.lda;
-  const long long lsb_c = g.transb ? 1 : g.ldb, lsb_k = g.transb ? g.ldb : 1;
+  const long long lsa_r = transa ? lda : 1, lsa_k = transa ? 1 : lda;
+  const long long lsb_c = transb ? 1 : ldb, lsb_k = transb ? ldb : 1;
   auto loadA = [&](int k0, S (&ra)[4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = row0 + ar[i], k = k0 + ak[i];
-      const int rc = r < g.M ? r : g.M - 1, kc = k < g.K ? k : g.K - 1;
+      const int rc = r < M ? r : M - 1, kc = k < K ? k : K - 1;
       ra[i] = A[rc * lsa_r + kc * lsa_k];
     }
   };
@@ -320,7 +298,7 @@ __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int c = col0 + bc[i], k = k0 + bk[i];
-      const int cc = c < g.N ? c : g.N - 1, kc = k < g.K ? k : g.K - 1;
+      const int cc = c < N ? c : N - 1, kc = k < K ? k : K - 1;
       rb[i] = B[cc * lsb_c + kc * lsb_k];
     }
   };
@@ -328,14 +306,13 @@ __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
                    Ls (*Bd)[GM_TILE + GM_PAD]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bool ina = row0 + ar[i] < g.M && k0 + ak[i] < g.K;
-      const bool inb = col0 + bc[i] < g.N && k0 + bk[i] < g.K;
+      const bool ina = row0 + ar[i] < M && k0 + ak[i] < K;
+      const bool inb = col0 + bc[i] < N && k0 + bk[i] < K;
       Ad[ak[i]][ar[i]] = TT::cvt(ina ? ra[i] : S(0));
       Bd[bk[i]][bc[i]] = TT::cvt(inb ? rb[i] : S(0));
     }
   };
 
-  v4 acc[2][2], acc2[2][2];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
@@ -370,10 +347,59 @@ __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     __syncthreads();
     cur ^= 1;
   };
-  for (int k0 = 0; k0 < g.K; k0 += 2 * GM_KC) {
+  for (int k0 = 0; k0 < K; k0 += 2 * GM_KC) {
     step(k0, ra0, rb0, ra1, rb1);
     step(k0 + GM_KC, ra1, rb1, ra0, rb0);
   }
+
+}
+
+// held to 128 registers (four waves per SIMD): with the second chunk buffer
+// the FP64 kind otherwise takes 136 and runs at three
+template <int KIND>
+__global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void eig_gemm_kernel(GemmArgs g)
+{
+  typedef GemmT<KIND> TT;
+  typedef typename TT::S S;
+  typedef typename TT::v4 v4;
+  __shared__ GemmLds<KIND> Sm;
+
+  const int tm = (g.M + GM_TILE - 1) / GM_TILE, tn = (g.N + GM_TILE - 1) / GM_TILE;
+  long long tiles;
+  int symw = g.sym;
+  if (symw > 0) {
+    // tn = nblk * symw tiles in blocks of symw x symw (tm == symw)
+    tiles = (long long)(tn / symw) * (symw * (symw + 1) / 2);
+  } else {
+    tiles = (long long)tm * tn;
+  }
+  const long long total = tiles * g.batch;
+  const long long lid = gemm_xcd_remap(blockIdx.x, total);
+  if (lid >= total) return;
+  const long long b = lid / tiles;
+  if (g.skip && g.skip[b] != 0) return;
+  int t = (int)(lid - b * tiles), ti, tj;
+  if (symw > 0) {
+    const int per = symw * (symw + 1) / 2;
+    const int blk = t / per;
+    int r = t - blk * per, J = 0;
+    while ((J + 1) * (J + 2) / 2 <= r) ++J;
+    ti = r - J * (J + 1) / 2;
+    tj = blk * symw + J;
+  } else {
+    ti = t % tm;
+    tj = t / tm;
+  }
+  const int row0 = ti * GM_TILE, col0 = tj * GM_TILE;
+  const S *__restrict__ A = (const S *)g.A + b * g.sa;
+  const S *__restrict__ B = (const S *)g.B + b * g.sb;
+
+  const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
+  const int m = lane & 15, gg = lane >> 4;
+  const int wr = (q & 1) * 32, wc = (q >> 1) * 32;
+
+  v4 acc[2][2], acc2[2][2];
+  gemm_tile<KIND>(g.M, g.N, g.K, g.transa, g.transb, A, g.lda, B, g.ldb, row0, col0, Sm, acc, acc2);
 
   // epilogue: C = alpha acc + beta D
   typedef typename TT::Acc Acc;

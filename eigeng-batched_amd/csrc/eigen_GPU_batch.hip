@@ -19,6 +19,7 @@
 #include "eig_split_large.hpp"
 #include "eig_tri_reg.hpp"
 #include "eig_dc.hpp"
+#include "eig_dc_large.hpp"
 #include "eig_check.hpp"
 #include "eig_symdmt.hpp"
 #include "eig_gemm.hpp"
@@ -219,6 +220,36 @@ bool use_dc(int L, int n, int tbytes, int solver)
   return n >= DC_MIN_N && L <= dc_max_l(n, tbytes) && (!(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L);
 }
 
+// 64 < n <= 512, the same interface.  FP32 n <= 128 batches of SPLIT_MIN_L
+// matrices and more keep the two-wave register tridiagonalisation with its
+// explicit Q, the others take reflectors and a blocked back-transformation.
+bool use_dc_large(int L, int n, int tbytes, int solver)
+{
+  (void)tbytes;
+  const int flags = solver & ~0xff & ~(3 << CHUNK_SHIFT) & ~FLAG_PH_ALL;
+  if ((solver & 0xff) != SOLVER_IMTQL2 || (flags & ~(FLAG_DC | FLAG_SPLIT)) || n <= 64 || n > GL_NMAX) return false;
+  return (flags & FLAG_DC) || !(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L;
+}
+bool dc_explicit_q(int L, int n, int tbytes) { return tbytes == 4 && n <= 128 && L >= SPLIT_MIN_L; }
+
+// Its workspace for a chunk of lc matrices: the reflectors (or Q), d / e, beta, two
+// buffers of eigenvectors of T, the merges' U (later the reflector blocks' T), status.
+struct DcLargeLayout {
+  size_t wm, de, bw, z0, z1, u, st, total;
+  DcLargeLayout(int lc, int n, int tb)
+  {
+    const size_t mat = al256((size_t)lc * n * n * tb);
+    wm = 0;
+    de = wm + mat;
+    bw = de + al256((size_t)2 * n * lc * tb);
+    z0 = bw + al256((size_t)lc * n * tb);
+    z1 = z0 + mat;
+    u = z1 + mat;
+    st = u + mat;
+    total = st + al256((size_t)lc * 4);
+  }
+};
+
 // Workspace of the divide and conquer path, n <= 64, for a chunk of lc matrices:
 // Q, d / e.
 struct DcLayout {
@@ -299,6 +330,11 @@ size_t workspace_bytes(int L, int nm, int n, int m, int tbytes, int solver)
     // that path fits in a workspace of the size the query reports
     const size_t other = workspace_bytes(L, nm, n, m, tbytes, (solver & ~FLAG_DC) | FLAG_ROUTE_QL);
     const size_t own = WS_HEAD + DcLayout(L < lchunk(solver) ? L : lchunk(solver), n, tbytes).total;
+    return own > other ? own : other;
+  }
+  if (use_dc_large(L, n, tbytes, solver)) {
+    const size_t other = workspace_bytes(L, nm, n, m, tbytes, (solver & ~FLAG_DC) | FLAG_ROUTE_QL);
+    const size_t own = WS_HEAD + DcLargeLayout(L < lchunk_large(solver) ? L : lchunk_large(solver), n, tbytes).total;
     return own > other ? own : other;
   }
   solver &= ~FLAG_ROUTE_QL;
@@ -384,7 +420,7 @@ void launch_dc_chunk(int cur, int nm, int n, T *a, T *w, int *info, int ph, int 
                        de, ld, UvSplitArgs{}, only);
   if (ph & FLAG_PH_APPLY)
     hipLaunchKernelGGL((eig_dc_kernel<T, NB, NLR, false>), dim3((unsigned)cur), dim3(NB * NLR), 0, s, cur, nm, n, a,
-                       (const T *)q, (const T *)de, ld, w, info, kop, nanfail, 1, (T *)nullptr, only);
+                       (const T *)q, (const T *)de, ld, w, info, kop, nanfail, 1, (T *)nullptr, (T *)nullptr, 0, only);
 }
 template <typename T>
 void dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, T *q, T *de, int ld,
@@ -915,6 +951,132 @@ int tuned_solver(int L, int n, int tb, int solver)
   return solver | bits;
 }
 
+// ---- divide and conquer, 64 < n <= 512 --------------------------------------------
+
+// The merge tree over nb blocks of 64 columns: lev[d] the merges at depth d (the
+// last one at depth 0); a node's vectors, blocks included, live in the buffer of
+// its depth's parity, so a merge reads one buffer and writes the other.  Returns
+// the number of levels; bit b of zmask: block b starts in buffer 1.
+void dc_tree(int n, int b0, int b1, int depth, DcNodes (&lev)[4], int &levels, int &zmask)
+{
+  if (b1 - b0 == 1) {
+    if (depth & 1) zmask |= 1 << b0;
+    return;
+  }
+  const int bm = b0 + (b1 - b0 + 1) / 2;
+  DcNodes &l = lev[depth];
+  l.base[l.cnt] = (short)(64 * b0);
+  l.mid[l.cnt] = (short)(64 * bm);
+  l.end[l.cnt] = (short)(64 * b1 < n ? 64 * b1 : n);
+  ++l.cnt;
+  if (depth + 1 > levels) levels = depth + 1;
+  dc_tree(n, b0, bm, depth + 1, lev, levels, zmask);
+  dc_tree(n, bm, b1, depth + 1, lev, levels, zmask);
+}
+
+template <typename T, int NT, int WPE>
+void launch_dc_back(int cur, int n, int nm, int mcols, const T *W, const T *Tm, const T *Z, T *a, const int *st,
+                    hipStream_t s)
+{
+  const int ncg = (mcols + 63) / 64;
+  hipLaunchKernelGGL((eig_dc_back_kernel<T, NT, WPE>), dim3((unsigned)cur * (unsigned)ncg), dim3(256), 0, s, cur, n,
+                     nm, mcols, ncg, W, Tm, Z, a, st);
+}
+
+// Phases: tridiagonalisation, tridiagonal eigenproblem, back-transformation.
+template <typename T>
+hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver, int kop, void *wk, hipStream_t s)
+{
+  constexpr int tb = (int)sizeof(T), KIND = tb == 8 ? GK_F64 : GK_F32;
+  const int lc = L < lchunk_large(solver) ? L : lchunk_large(solver);
+  const DcLargeLayout lay(lc, n, tb);
+  char *base = (char *)wk + WS_HEAD;
+  T *Wm = (T *)(base + lay.wm), *de = (T *)(base + lay.de), *bw = (T *)(base + lay.bw), *U = (T *)(base + lay.u);
+  T *Z[2] = {(T *)(base + lay.z0), (T *)(base + lay.z1)};
+  int *st = (int *)(base + lay.st);
+  const int ph = (solver & FLAG_PH_ALL) ? (solver & FLAG_PH_ALL) : FLAG_PH_ALL;
+  if (ph != FLAG_PH_ALL && L > lc) return hipErrorInvalidValue;
+  const bool xq = dc_explicit_q(L, n, tb);
+  const int nanfail = L < (tb == 4 && n <= 128 ? SPLIT_MIN_L : SPLIT_LARGE_MIN_L) ? 1 : 0;
+  const int nblk = (n + 63) / 64, nb16 = (n + 15) / 16, mcols = n - kopt_mdrop(kop);
+  DcNodes lev[4] = {};
+  int levels = 0, zmask = 0;
+  dc_tree(n, 0, nblk, 0, lev, levels, zmask);
+  for (long long c0 = 0; c0 < L; c0 += lc) {
+    const int cur = (int)((L - c0) < lc ? (L - c0) : lc);
+    T *ac = a + (size_t)c0 * nm * n;
+    T *wc = w + (size_t)c0 * n;
+    int *ic = info ? info + c0 : nullptr;
+    const unsigned tg = (unsigned)(cur < 1024 ? cur : 1024);
+    if (ph & FLAG_PH_TRI) {
+      if (xq) {
+        if constexpr (tb == 4)
+          hipLaunchKernelGGL((eig_tri_kernel<T, 128>), dim3((unsigned)cur), dim3(128), 0, s, cur, nm, n, (const T *)ac,
+                             Wm, de, lc, UvSplitArgs{}, (const int *)nullptr);
+      } else if (n <= 128) {
+        hipLaunchKernelGGL((eig_tri_reg_kernel<T, 4, 3, 3>), dim3(tg), dim3(256), 0, s, cur, nm, n, (const T *)ac, Wm,
+                           de, lc, bw);
+      } else if (n <= 256) {
+        hipLaunchKernelGGL((eig_tri_reg_kernel<T, 12, 3, 3>), dim3(tg), dim3(768), 0, s, cur, nm, n, (const T *)ac,
+                           Wm, de, lc, bw);
+      } else {
+        hipLaunchKernelGGL((eig_tri_large_kernel<T, 256, 8, 512, 1>), dim3(tg), dim3(256), 0, s, cur, nm, n,
+                           (const T *)ac, Wm, de, lc, bw);
+      }
+    }
+    if (ph & FLAG_PH_QL) {
+      hipLaunchKernelGGL((eig_dc_kernel<T, 64, 4, true>), dim3((unsigned)cur * (unsigned)nblk), dim3(256), 0, s, cur,
+                         n, n, (T *)nullptr, (const T *)nullptr, (const T *)de, lc, wc, (int *)nullptr, kop, 0, nblk,
+                         Z[0], Z[1], zmask, (const int *)nullptr);
+      for (int d = levels - 1; d >= 0; --d) {
+        const DcNodes &l = lev[d];
+        int big = 0, tiles = 0;
+        for (int q = 0; q < l.cnt; ++q) {
+          const int sz = l.end[q] - l.base[q], nt = (sz + 63) / 64;
+          big = sz > big ? sz : big;
+          tiles += nt * nt;
+        }
+        const unsigned grid = (unsigned)cur * (unsigned)l.cnt;
+        const T *Zc = Z[(d + 1) & 1];
+        int *sd = d == 0 ? st : nullptr;
+        if (big <= 128)
+          hipLaunchKernelGGL((eig_dc_merge_kernel<T, 128, 4>), dim3(grid), dim3(512), 0, s, n, l, (const T *)de, lc, wc,
+                             Zc, U, sd, ic, nanfail);
+        else if (big <= 256)
+          hipLaunchKernelGGL((eig_dc_merge_kernel<T, 256, 4>), dim3(grid), dim3(1024), 0, s, n, l, (const T *)de, lc,
+                             wc, Zc, U, sd, ic, nanfail);
+        else
+          hipLaunchKernelGGL((eig_dc_merge_kernel<T, 512, 2>), dim3(grid), dim3(1024), 0, s, n, l, (const T *)de, lc,
+                             wc, Zc, U, sd, ic, nanfail);
+        hipLaunchKernelGGL((eig_dc_update_kernel<T>), dim3((unsigned)cur * (unsigned)tiles), dim3(GM_THREADS), 0, s,
+                           cur, n, l, tiles, Zc, (const T *)U, Z[d & 1]);
+      }
+    }
+    if (ph & FLAG_PH_APPLY) {
+      if (xq) {
+        GemmArgs g{};
+        const long long nn = (long long)n * n;
+        g.M = n; g.N = mcols; g.K = n; g.batch = cur; g.alpha = 1.0; g.skip = st;
+        g.A = Wm; g.lda = n; g.sa = nn;
+        g.B = Z[0]; g.ldb = n; g.sb = nn;
+        g.C = ac; g.ldc = nm; g.sc = (long long)nm * n;
+        const hipError_t err = gemm_launch(KIND, g, s);
+        if (err != hipSuccess) return err;
+      } else {
+        const long long blocks = (long long)cur * nb16;
+        hipLaunchKernelGGL((eig_dc_wyt_kernel<T>), dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, blocks, n,
+                           nb16, (const T *)Wm, (const T *)bw, U);
+        constexpr int W8 = tb == 8 ? 3 : 4, W16 = tb == 8 ? 2 : 3, W24 = tb == 8 ? 2 : 3, W32 = tb == 8 ? 1 : 2;
+        if (n <= 128) launch_dc_back<T, 8, W8>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+        else if (n <= 256) launch_dc_back<T, 16, W16>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+        else if (n <= 384) launch_dc_back<T, 24, W24>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+        else launch_dc_back<T, 32, W32>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+      }
+    }
+  }
+  return hipGetLastError();
+}
+
 template <typename T>
 hipError_t run(int L, int nm, int n, int m, T *a, T *w, void *wk, hipStream_t s, int solver, int *info)
 {
@@ -931,6 +1093,7 @@ hipError_t run(int L, int nm, int n, int m, T *a, T *w, void *wk, hipStream_t s,
   // kernel options: solver, order of the output, eigenvector columns not stored
   const int kop = kopt_make(base, (solver & FLAG_UNSORTED) != 0, n - m);
   if (use_dc(L, n, (int)sizeof(T), solver)) return run_dc<T>(L, nm, n, a, w, info, solver, kop, wk, s);
+  if (use_dc_large(L, n, (int)sizeof(T), solver)) return run_dc_large<T>(L, nm, n, a, w, info, solver, kop, wk, s);
   if ((solver & FLAG_PH_ALL) && !use_split(L, n, (int)sizeof(T), solver) && !use_split_large(L, n, (int)sizeof(T), solver) &&
       !use_split128(L, n, (int)sizeof(T), solver))
     return hipErrorInvalidValue;
@@ -980,6 +1143,7 @@ std::vector<int> tune_candidates(int L, int n, int tb, int solver)
       c.push_back(FLAG_SPLIT | (1 << CHUNK_SHIFT));
       return c;
     }
+    if (base == SOLVER_IMTQL2) c.push_back(FLAG_DC);
     c.push_back(FLAG_REG128);
     c.push_back(FLAG_SPLIT | (1 << TRI_CFG_SHIFT));
     c.push_back(FLAG_SPLIT | (2 << TRI_CFG_SHIFT));
@@ -987,6 +1151,7 @@ std::vector<int> tune_candidates(int L, int n, int tb, int solver)
     return c;
   }
   if (n > GL_NMAX) return c;
+  if (base == SOLVER_IMTQL2) c.push_back(FLAG_DC);
   c.push_back(FLAG_FUSED | (1 << GL_NT_SHIFT));
   c.push_back(FLAG_FUSED | (2 << GL_NT_SHIFT));
   // tridiagonalisation shapes: symmetric form 256 / 512 threads and the full
@@ -1722,6 +1887,13 @@ hipError_t launch_params(int L, int n, int tb, int solver, int *p)
   };
   if (use_dc(L, n, tb, solver)) {
     grp(nb_of(n), L < lchunk(solver) ? L : lchunk(solver), 64);
+  } else if (use_dc_large(L, n, tb, solver)) {
+    const int lc = L < lchunk_large(solver) ? L : lchunk_large(solver);
+    if (dc_explicit_q(L, n, tb)) {
+      grp(128, lc, 128);
+    } else {
+      p[0] = 256; p[1] = lc < 1024 ? lc : 1024; p[2] = 1; p[3] = 256;
+    }
   } else if (tb == 4 && use_split128(L, n, tb, solver)) {
     grp(128, L < lchunk(solver) ? L : lchunk(solver), 128);
   } else if (use_split(L, n, tb, solver)) {

@@ -68,14 +68,44 @@ def test_families(n, dtype, reps):
     check(a, z[:, :, :n], w.cpu().numpy(), dtype)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [65, 66, 128, 129, 192, 193, 256, 257, 320, 321, 384, 385, 449, 512])
+def test_families_of_several_blocks(n, dtype):
+    """Every shape of the merge tree over blocks of 64 columns (one column in the
+    last block, full blocks, uneven halves) and every back-transformation size."""
+    print(f"[dc] n={n} {np.dtype(dtype).name}", flush=True)
+    a = families(n, np.random.default_rng(n)).astype(dtype)
+    t = torch.full((a.shape[0], n, n + 1), float("nan"), dtype=torch.float32 if dtype == np.float32 else torch.float64)
+    t[:, :, :n] = torch.from_numpy(np.tril(a))
+    z, w, info = eg.eigen_batch(t.to(DEV), path="dc")
+    torch.cuda.synchronize()
+    assert int(info.abs().max()) == 0
+    z = z.cpu().numpy()
+    assert np.isnan(z[:, :, n:]).all()
+    check(a, z[:, :, :n], w.cpu().numpy(), dtype)
+
+
+@pytest.mark.parametrize("n", [65, 100, 128])
+def test_families_with_explicit_q(n):
+    """FP32 batches of 2048 and more, n <= 128: Q formed by the tridiagonalisation
+    and multiplied; the same bound, and the small batch's eigenvalues."""
+    a = np.tile(families(n, np.random.default_rng(n)).astype(np.float32), (130, 1, 1))
+    t = torch.from_numpy(np.tril(a)).to(DEV)
+    z, w, info = eg.eigen_batch(t.clone())
+    torch.cuda.synchronize()
+    assert int(info.abs().max()) == 0
+    check(a, z.cpu().numpy(), w.cpu().numpy(), np.float32)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("n", [8, 33, 64])
+@pytest.mark.parametrize("n", [8, 33, 64, 100, 130, 300])
 def test_first_columns_and_smaller_chunks(n, dtype):
     """m < n stores the same first columns and eigenvalues; a divided chunk and a
     call phase by phase give the same bits."""
     g = torch.Generator(device=DEV)
     g.manual_seed(n)
-    b = torch.rand((900, n, n), generator=g, device=DEV, dtype=dtype) - 0.5
+    L = 900 if n <= 130 else 20
+    b = torch.rand((L, n, n), generator=g, device=DEV, dtype=dtype) - 0.5
     a = (b + b.transpose(1, 2)).contiguous()
     z, w, _ = eg.eigen_batch(a.clone(), path="dc")
     m = n // 2
@@ -83,15 +113,16 @@ def test_first_columns_and_smaller_chunks(n, dtype):
     assert torch.equal(w, wm) and torch.equal(z[:, :m], zm[:, :m]) and torch.equal(zm[:, m:], a[:, m:])
     zc, wc, _ = eg.eigen_batch(a.clone(), solver=eg.IMTQL2 | (3 << eg.CHUNK_SHIFT), path="dc")
     assert torch.equal(w, wc) and torch.equal(z, zc)
-    ws = torch.empty(eg.bufsize(900, n, n, n, a.element_size(), eg.FLAG_DC), dtype=torch.uint8, device=DEV)
-    zp, wp, info = a.clone(), torch.empty_like(w), torch.empty(900, dtype=torch.int32, device=DEV)
+    ws = torch.empty(eg.bufsize(L, n, n, n, a.element_size(), eg.FLAG_DC), dtype=torch.uint8, device=DEV)
+    zp, wp, info = a.clone(), torch.empty_like(w), torch.empty(L, dtype=torch.int32, device=DEV)
     for ph in ("tri", "ql", "apply"):
         eg.eigen_batch(zp, w=wp, info=info, workspace=ws, path="dc", phases=[ph])
     assert torch.equal(w, wp) and torch.equal(z, zp)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("n,L", [(20, 40), (20, 3000), (48, 100), (48, 2100), (64, 30)])
+@pytest.mark.parametrize("n,L", [(20, 40), (20, 3000), (48, 100), (48, 2100), (64, 30), (100, 60), (100, 2050),
+                                 (200, 30), (200, 520)])
 def test_matrices_that_are_not_finite(n, L, dtype):
     """A NaN or an infinity in one matrix: the status of the path the batch took
     before (the fused kernel's for small batches, the split path's for large ones),
@@ -105,10 +136,19 @@ def test_matrices_that_are_not_finite(n, L, dtype):
     a[1, :, :] = float("nan")
     a[7, 5, 3] = float("nan")
     a[20, 4, 4] = float("inf")
-    small = n not in (20,) and L < 2048 or (n == 20 and dtype == torch.float32 and L < 2048)
+    small = n not in (20,) and n < 65 and L < 2048 or (n == 20 and dtype == torch.float32 and L < 2048)
     if dtype == torch.float32 and n == 64:
         small = L < 1024
     z, w, info = eg.eigen_batch(a.clone())
+    if n > 64:
+        # the same statuses: 1 from the small batch's path, 0 from the large one's
+        small = L < (2048 if dtype == torch.float32 and n <= 128 else 512)
+        ok = [k for k in range(L) if k not in bad]
+        assert torch.equal(z[ok], good[ok]) and torch.equal(w[ok], gw[ok]) and int(info[ok].abs().max()) == 0
+        for k in bad:
+            assert int(info[k]) == (1 if small else 0) and bool(torch.isnan(w[k]).any())
+            assert bool(torch.isnan(z[k]).any()) or (small and torch.equal(z[k], a[k]))
+        return
     zq, wq, iq = eg.eigen_batch(a.clone(), path="fused" if small else "split")
     ok = [k for k in range(L) if k not in bad]
     assert torch.equal(info, iq)
