@@ -33,6 +33,13 @@ __device__ __forceinline__ void wsync()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Workgroup barrier that orders LDS traffic only: global loads and stores in
+// flight are not waited for (__syncthreads waits for them).
+__device__ __forceinline__ void lds_barrier()
+{
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ---- raw 32-bit lane movement -------------------------------------------
 template <int CTRL>
 __device__ __forceinline__ int dpp32(int x)
@@ -305,6 +312,18 @@ __device__ __forceinline__ double swap_sum(double a, double b)
   const unsigned ahi = swap_u32<W>((unsigned)(ab >> 32), (unsigned)(bb >> 32), bhi);
   return __longlong_as_double((long long)(((unsigned long long)ahi << 32) | alo)) +
          __longlong_as_double((long long)(((unsigned long long)bhi << 32) | blo));
+}
+
+// Sum over the 64 lanes of a wave on the VALU alone (the same in every lane).
+template <typename T>
+__device__ __forceinline__ T wave_sum(T x)
+{
+  x += lane_move(x, MvX1());
+  x += lane_move(x, MvX2());
+  x += lane_move(x, MvHM());
+  x += lane_move(x, MvRM());
+  x = swap_sum<16>(x, x);
+  return swap_sum<32>(x, x);
 }
 
 } // namespace eigmi

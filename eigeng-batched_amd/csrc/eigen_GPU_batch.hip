@@ -18,6 +18,7 @@
 #include "eig_uneven.hpp"
 #include "eig_split_large.hpp"
 #include "eig_tri_reg.hpp"
+#include "eig_tri_stream.hpp"
 #include "eig_dc.hpp"
 #include "eig_dc_large.hpp"
 #include "eig_check.hpp"
@@ -1020,8 +1021,10 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
         hipLaunchKernelGGL((eig_tri_reg_kernel<T, 12, 3, 3>), dim3(tg), dim3(768), 0, s, cur, nm, n, (const T *)ac,
                            Wm, de, lc, bw);
       } else {
-        hipLaunchKernelGGL((eig_tri_large_kernel<T, 256, 8, 512, 1>), dim3(tg), dim3(256), 0, s, cur, nm, n,
-                           (const T *)ac, Wm, de, lc, bw);
+        // the strips in the first buffer of vectors, which is free until the merges
+        constexpr int NBP = tb == 8 ? 8 : 16, NT = tb == 8 ? 512 : 1024;
+        hipLaunchKernelGGL((eig_tri_stream_kernel<T, NBP, NT>), dim3(tg), dim3(NT), 0, s, cur, nm, n, (const T *)ac,
+                           Wm, Z[0], (long long)ts_strips(n) * 1024, de, lc, bw);
       }
     }
     if (ph & FLAG_PH_QL) {

@@ -85,6 +85,21 @@ def test_families_of_several_blocks(n, dtype):
     check(a, z[:, :, :n], w.cpu().numpy(), dtype)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [257, 264, 272])
+def test_more_matrices_than_workgroups(n, dtype):
+    """Above 1024 matrices a workgroup of the tridiagonalisation takes a second one:
+    copies of one matrix give the same bits wherever they stand in the batch."""
+    a = families(n, np.random.default_rng(n))[:5].astype(dtype)
+    z0, w0, _ = eg.eigen_batch(torch.from_numpy(np.tril(a)).to(DEV), path="dc")
+    check(a, z0.cpu().numpy(), w0.cpu().numpy(), dtype)
+    z, w, info = eg.eigen_batch(torch.from_numpy(np.tril(a)).to(DEV).repeat(206, 1, 1), path="dc")
+    torch.cuda.synchronize()
+    assert int(info.abs().max()) == 0
+    assert torch.equal(z.view(206, *z0.shape), z0.expand(206, *z0.shape))
+    assert torch.equal(w.view(206, *w0.shape), w0.expand(206, *w0.shape))
+
+
 @pytest.mark.parametrize("n", [65, 100, 128])
 def test_families_with_explicit_q(n):
     """FP32 batches of 2048 and more, n <= 128: Q formed by the tridiagonalisation
