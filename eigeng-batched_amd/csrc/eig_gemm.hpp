@@ -247,7 +247,8 @@ __device__ __forceinline__ long long gemm_xcd_remap(long long bid, long long tot
 // chunk.  Non-transposed A (rows contiguous): thread t takes row t & 63 and k =
 // (t >> 6) + 4 i; transposed A (k contiguous): k = t & 15, row = (t >> 4) + 16 i.
 // B likewise with the roles of rows and k exchanged.  acc (and acc2 for GK_F16X3):
-// wave q's 32 x 32 quarter of the tile at (row0, col0) of op(A) op(B).
+// wave q's 32 x 32 quarter of the tile at (row0, col0) of op(A) op(B), or of
+// op(A) diag(dk) op(B) with DIAG (dk in LDS, readable to index K + 47).
 template <int KIND>
 struct alignas(16) GemmLds {
   // two chunk buffers: the next chunk is stored while the current one is
@@ -255,12 +256,13 @@ struct alignas(16) GemmLds {
   typename GemmT<KIND>::L A[2][GM_KC][GM_TILE + GM_PAD];
   typename GemmT<KIND>::L B[2][GM_KC][GM_TILE + GM_PAD];
 };
-template <int KIND>
+template <int KIND, bool DIAG = false>
 __device__ __forceinline__ void gemm_tile(int M, int N, int K, int transa, int transb,
                                           const typename GemmT<KIND>::S *__restrict__ A, long long lda,
                                           const typename GemmT<KIND>::S *__restrict__ B, long long ldb, int row0,
                                           int col0, GemmLds<KIND> &Sm, typename GemmT<KIND>::v4 (&acc)[2][2],
-                                          typename GemmT<KIND>::v4 (&acc2)[2][2])
+                                          typename GemmT<KIND>::v4 (&acc2)[2][2],
+                                          const typename GemmT<KIND>::S *dk = nullptr)
 {
   typedef GemmT<KIND> TT;
   typedef typename TT::S S;
@@ -308,7 +310,9 @@ __device__ __forceinline__ void gemm_tile(int M, int N, int K, int transa, int t
     for (int i = 0; i < 4; ++i) {
       const bool ina = row0 + ar[i] < M && k0 + ak[i] < K;
       const bool inb = col0 + bc[i] < N && k0 + bk[i] < K;
-      Ad[ak[i]][ar[i]] = TT::cvt(ina ? ra[i] : S(0));
+      S va = ra[i];
+      if constexpr (DIAG) va *= dk[k0 + ak[i]];
+      Ad[ak[i]][ar[i]] = TT::cvt(ina ? va : S(0));
       Bd[bk[i]][bc[i]] = TT::cvt(inb ? rb[i] : S(0));
     }
   };

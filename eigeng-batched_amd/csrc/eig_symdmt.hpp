@@ -1,7 +1,7 @@
 // eig_symdmt.hpp - the dense batched products on either side of the solver, on
 // MFMA (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64, FP32 / FP64 accumulate):
 //
-//   eig_symdmt_kernel  C_k = Z_k diag(d_k) Z_k^T, with d_k given or
+//   eig_symdmt_*       C_k = Z_k diag(d_k) Z_k^T, with d_k given or
 //                      d_k = scale * w_k^p (the LETKF consumer step: the analysis
 //                      covariance V L^-1 V^T, the transform sqrt(k-1) V L^-1/2 V^T).
 //                      Reference: the batched symdmt_batch experiment (symdmt.cu:5-87)
@@ -10,16 +10,19 @@
 //                      LETKF ingest that forms the matrices the solver takes;
 //                      the reference forms its inputs on the host, main.cpp:63-195).
 //
-// Both outputs are symmetric: a workgroup owns one matrix and its waves take the
-// 32 x 32 output blocks (I, J), I <= J, in turn; a block is 2 x 2 MFMA tiles of
-// 16 x 16 accumulated over the contraction in steps of 4.  Every block value is
-// written to both (i, j) and (j, i), so the result is exactly symmetric.
+// Both outputs are symmetric: only tiles (I, J), I <= J, are formed and every value
+// is written to both (i, j) and (j, i), so the result is exactly symmetric.  n <= 64:
+// one wave per matrix.  n > 64: eig_symdmt_tile_kernel takes 64 x 64 tiles of all
+// matrices; in eig_gram_kernel a workgroup owns one matrix and its waves take the
+// 32 x 32 output blocks in turn, 2 x 2 MFMA tiles of 16 x 16 accumulated over the
+// contraction in steps of 4.
 //
 // MFMA operand layout (16x16x4, wave64): lane l = m + 16 g holds A(m, g) and
 // B(g, m); accumulator slot r of lane l holds C(row(g, r), m) with
 // row = 4 g + r for f32 and g + 4 r for f64.
 #pragma once
 #include "common.hpp"
+#include "eig_gemm.hpp"
 #include "eig_global.hpp"
 
 namespace eigmi {
@@ -91,50 +94,49 @@ __device__ __forceinline__ T dfun(T w, int fn, T p, T scale)
   return scale * v;
 }
 
+// n > 64: a workgroup per 64 x 64 tile (ti, tj), ti <= tj, of one product, the
+// operands through LDS with the diagonal multiplied in on the way.  FP64 is bound by
+// the matrix cores (n = 256: ten tiles of 2 64 64 256 operations per matrix, 2.4 ms of
+// the 3.9 that 8192 products take), FP32 by memory (n = 128: 0.23 of 0.46 ms).  One
+// workgroup per matrix with operands straight from L2 took 11.1 and 0.83 ms, and left
+// the chip idle where the batch is small: 64 products of n = 512 in FP64 4.70 ms,
+// 0.24 ms now; 160 of n = 120 in FP32 14 us.
 template <typename T>
-__global__ __launch_bounds__(SD_MAX_THREADS) void eig_symdmt_kernel(int L, int nm, int n, const T *__restrict__ z,
-                                                                    const T *__restrict__ dsrc, int fn, T p,
-                                                                    T scale, T *__restrict__ out)
+__global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void eig_symdmt_tile_kernel(
+    int L, int nm, int n, const T *__restrict__ z, const T *__restrict__ dsrc, int fn, T p, T scale,
+    T *__restrict__ out)
 {
-  typedef typename Mfma16<T>::v4 v4;
-  __shared__ T ds[GL_NMAX];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, nw = blockDim.x >> 6;
-  const int m = lane & 15, g = lane >> 4;
-  const int nb = (n + 31) >> 5, nblk = nb * (nb + 1) / 2;
-  for (long long mat = blockIdx.x; mat < L; mat += gridDim.x) {
+  constexpr int KIND = sizeof(T) == 8 ? GK_F64 : GK_F32;
+  __shared__ GemmLds<KIND> Sm;
+  __shared__ T ds[GL_NMAX + GM_TILE];
+  const int tm = (n + GM_TILE - 1) / GM_TILE, tiles = tm * (tm + 1) / 2;
+  const long long total = (long long)tiles * L;
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, m = lane & 15, g = lane >> 4;
+  const int wr = (q & 1) * 32, wc = (q >> 1) * 32;
+  for (long long bid = blockIdx.x; bid < total; bid += gridDim.x) {
+    const long long lid = gemm_xcd_remap(bid, total), mat = lid / tiles;
+    int ti, tj;
+    sym_block((int)(lid - mat * tiles), ti, tj);
     const T *__restrict__ Z = z + (size_t)mat * nm * n;
     const T *__restrict__ D = dsrc + (size_t)mat * n;
     T *__restrict__ O = out + (size_t)mat * nm * n;
-    for (int i = t; i < n; i += blockDim.x) ds[i] = dfun(D[i], fn, p, scale);
+    for (int i = threadIdx.x; i < n + GM_TILE; i += GM_THREADS) ds[i] = i < n ? dfun(D[i], fn, p, scale) : T(0);
     __syncthreads();
-    for (int blk = wv; blk < nblk; blk += nw) {
-      int I, J;
-      sym_block(blk, I, J);
-      // operand rows (clamped into the matrix; rows >= n only feed outputs
-      // that are not stored)
-      const int ra0 = min(32 * I + m, n - 1), ra1 = min(32 * I + 16 + m, n - 1);
-      const int rb0 = min(32 * J + m, n - 1), rb1 = min(32 * J + 16 + m, n - 1);
-      v4 acc[2][2];
+    typename GemmT<KIND>::v4 acc[2][2], acc2[2][2];
+    gemm_tile<KIND, true>(n, n, n, 0, 1, Z, nm, Z, nm, GM_TILE * ti, GM_TILE * tj, Sm, acc, acc2, ds);
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = v4{0, 0, 0, 0};
-#pragma unroll 4
-      for (int k0 = 0; k0 < n; k0 += 4) {
-        const int k = k0 + g;
-        const bool kv = k < n;
-        const T *__restrict__ col = Z + (size_t)(kv ? k : n - 1) * nm;
-        const T dk = kv ? ds[k] : T(0);
-        const T a0 = kv ? col[ra0] * dk : T(0), a1 = kv ? col[ra1] * dk : T(0);
-        const T b0 = col[rb0], b1 = col[rb1];
-        acc[0][0] = Mfma16<T>::op(a0, b0, acc[0][0]);
-        acc[0][1] = Mfma16<T>::op(a0, b1, acc[0][1]);
-        acc[1][0] = Mfma16<T>::op(a1, b0, acc[1][0]);
-        acc[1][1] = Mfma16<T>::op(a1, b1, acc[1][1]);
-      }
-      store_sym_block<T>(O, nm, n, I, J, acc, T(0));
-    }
-    __syncthreads();
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = GM_TILE * ti + wr + 16 * x + GemmMma<KIND>::row(g, r);
+          const int j = GM_TILE * tj + wc + 16 * y + m;
+          if (i < n && j < n && i <= j) {
+            O[j + (size_t)i * nm] = acc[x][y][r];           // lanes m: consecutive rows of column i
+            O[i + (size_t)j * nm] = acc[x][y][r];
+          }
+        }
   }
 }
 

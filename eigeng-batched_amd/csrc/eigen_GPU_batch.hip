@@ -1827,9 +1827,10 @@ hipError_t run_symdmt(int L, int nm, int n, const T *z, const T *d, int fn, T p,
     }
     return hipGetLastError();
   }
-  const unsigned grid = (unsigned)(L < 4096 ? L : 4096);
-  hipLaunchKernelGGL((eig_symdmt_kernel<T>), dim3(grid), dim3(sd_threads(n)), 0, s, L, nm, n, z, d, fn, p, scale,
-                     c);
+  const int tm = (n + GM_TILE - 1) / GM_TILE;
+  const long long tiles = (long long)L * (tm * (tm + 1) / 2);
+  const unsigned grid = (unsigned)(tiles < 4000000 ? tiles : 4000000);      // of 256 threads: below 2^32 in all
+  hipLaunchKernelGGL((eig_symdmt_tile_kernel<T>), dim3(grid), dim3(GM_THREADS), 0, s, L, nm, n, z, d, fn, p, scale, c);
   return hipGetLastError();
 }
 
