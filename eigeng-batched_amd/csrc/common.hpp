@@ -326,4 +326,39 @@ __device__ __forceinline__ T wave_sum(T x)
   return swap_sum<32>(x, x);
 }
 
+// ---- products with a value of another lane of the row -------------------------
+// The FMA units take one operand from a fixed lane of the reader's row of 16 lanes
+// (DPP row_newbcast), so 16 values held by the 16 lanes of a row multiply without
+// LDS reads: s0 + s1 += sum_k x[lane k of the row] a[k].  Written as one block: the
+// compiler does not fold the lane move into the FMA and knows no hazard inside, so
+// the two wait states between a write of x and its first use are in the block.
+#define EIGMI_BC(op, d, x, a, k) "v_fmac_" op "_dpp %" #d ", %" #x ", %" #a " row_newbcast:" #k " row_mask:0xf bank_mask:0xf\n\t"
+#define EIGMI_DOT16(op)                                                                                           \
+  asm("s_nop 1\n\t" EIGMI_BC(op, 0, 2, 3, 0) EIGMI_BC(op, 1, 2, 4, 1) EIGMI_BC(op, 0, 2, 5, 2)                   \
+      EIGMI_BC(op, 1, 2, 6, 3) EIGMI_BC(op, 0, 2, 7, 4) EIGMI_BC(op, 1, 2, 8, 5) EIGMI_BC(op, 0, 2, 9, 6)         \
+      EIGMI_BC(op, 1, 2, 10, 7) EIGMI_BC(op, 0, 2, 11, 8) EIGMI_BC(op, 1, 2, 12, 9) EIGMI_BC(op, 0, 2, 13, 10)    \
+      EIGMI_BC(op, 1, 2, 14, 11) EIGMI_BC(op, 0, 2, 15, 12) EIGMI_BC(op, 1, 2, 16, 13)                            \
+      EIGMI_BC(op, 0, 2, 17, 14) EIGMI_BC(op, 1, 2, 18, 15)                                                       \
+      : "+v"(s0), "+v"(s1)                                                                                        \
+      : "v"(x), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),           \
+        "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]), "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15]))
+__device__ __forceinline__ void bcast_dot16(const float (&a)[16], float x, float &s0, float &s1) { EIGMI_DOT16("f32"); }
+__device__ __forceinline__ void bcast_dot16(const double (&a)[16], double x, double &s0, double &s1)
+{
+  EIGMI_DOT16("f64");
+}
+// a[k] += x[lane k of the row] y
+#define EIGMI_AXPY16(op)                                                                                          \
+  asm("s_nop 1\n\t" EIGMI_BC(op, 0, 16, 17, 0) EIGMI_BC(op, 1, 16, 17, 1) EIGMI_BC(op, 2, 16, 17, 2)             \
+      EIGMI_BC(op, 3, 16, 17, 3) EIGMI_BC(op, 4, 16, 17, 4) EIGMI_BC(op, 5, 16, 17, 5)                            \
+      EIGMI_BC(op, 6, 16, 17, 6) EIGMI_BC(op, 7, 16, 17, 7) EIGMI_BC(op, 8, 16, 17, 8)                            \
+      EIGMI_BC(op, 9, 16, 17, 9) EIGMI_BC(op, 10, 16, 17, 10) EIGMI_BC(op, 11, 16, 17, 11)                        \
+      EIGMI_BC(op, 12, 16, 17, 12) EIGMI_BC(op, 13, 16, 17, 13) EIGMI_BC(op, 14, 16, 17, 14)                      \
+      EIGMI_BC(op, 15, 16, 17, 15)                                                                                \
+      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),           \
+        "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15])      \
+      : "v"(x), "v"(y))
+__device__ __forceinline__ void bcast_axpy16(float (&a)[16], float x, float y) { EIGMI_AXPY16("f32"); }
+__device__ __forceinline__ void bcast_axpy16(double (&a)[16], double x, double y) { EIGMI_AXPY16("f64"); }
+
 } // namespace eigmi

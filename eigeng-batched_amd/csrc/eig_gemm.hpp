@@ -61,7 +61,6 @@ struct GemmArgs {
   void *C; long long ldc, sc;
   double alpha, beta;
   int sym;                              // 0, or the width (in 64-wide tiles) of the symmetric blocks
-  const int *skip;                      // may be null: products b with skip[b] != 0 are left out
 };
 
 constexpr int GM_TILE = 64, GM_KC = 16, GM_THREADS = 256, GM_PAD = 4;
@@ -381,7 +380,6 @@ __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   const long long lid = gemm_xcd_remap(blockIdx.x, total);
   if (lid >= total) return;
   const long long b = lid / tiles;
-  if (g.skip && g.skip[b] != 0) return;
   int t = (int)(lid - b * tiles), ti, tj;
   if (symw > 0) {
     const int per = symw * (symw + 1) / 2;

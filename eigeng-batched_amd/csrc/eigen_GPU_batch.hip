@@ -221,9 +221,9 @@ bool use_dc(int L, int n, int tbytes, int solver)
   return n >= DC_MIN_N && L <= dc_max_l(n, tbytes) && (!(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L);
 }
 
-// 64 < n <= 512, the same interface.  FP32 n <= 128 batches of SPLIT_MIN_L
-// matrices and more keep the two-wave register tridiagonalisation with its
-// explicit Q, the others take reflectors and a blocked back-transformation.
+// 64 < n <= 512, the same interface: reflectors and a blocked back-transformation.
+// (FP32 n = 128, 8192 matrices: the two-wave tridiagonalisation that forms Q and a
+// product with it take 3.95 + 0.72 ms, reflectors 2.06 + 1.14.)
 bool use_dc_large(int L, int n, int tbytes, int solver)
 {
   (void)tbytes;
@@ -231,7 +231,6 @@ bool use_dc_large(int L, int n, int tbytes, int solver)
   if ((solver & 0xff) != SOLVER_IMTQL2 || (flags & ~(FLAG_DC | FLAG_SPLIT)) || n <= 64 || n > GL_NMAX) return false;
   return (flags & FLAG_DC) || !(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L;
 }
-bool dc_explicit_q(int L, int n, int tbytes) { return tbytes == 4 && n <= 128 && L >= SPLIT_MIN_L; }
 
 // Its workspace for a chunk of lc matrices: the reflectors (or Q), d / e, beta, two
 // buffers of eigenvectors of T, the merges' U (later the reflector blocks' T), status.
@@ -586,6 +585,25 @@ hipError_t wy_backtransform(int cur, int nm, int n, float *Wm, const float *bw, 
   return hipSuccess;
 }
 
+// Register-resident tridiagonalisation, n <= 256.  For 128 < n <= 192 two (FP32: three)
+// matrices fit in a compute unit with four waves each, which pays once there are more
+// matrices than compute units (256): n = 160, FP64, 320 matrices 461 us against 671 in
+// eight waves; 256 matrices 350 against 349, FP32 at n = 192 384 against 332.  By L, not
+// by the chunk, so that a divided batch gives the same bits.
+template <typename T>
+void launch_tri_reg(int L, int cur, int nm, int n, const T *a, T *W, T *de, int ld, T *bw, unsigned grid, hipStream_t s)
+{
+  constexpr bool dp = sizeof(T) == 8;
+  if (n <= 128)
+    hipLaunchKernelGGL((eig_tri_reg_kernel<T, 2, 4, dp ? 3 : 4>), dim3(grid), dim3(256), 0, s, cur, nm, n, a, W, de,
+                       ld, bw);
+  else if (n <= 192 && L > 256)
+    hipLaunchKernelGGL((eig_tri_reg_kernel<T, 3, 4, dp ? 2 : 3>), dim3(grid), dim3(256), 0, s, cur, nm, n, a, W, de,
+                       ld, bw);
+  else
+    hipLaunchKernelGGL((eig_tri_reg_kernel<T, 4, 8, 2>), dim3(grid), dim3(512), 0, s, cur, nm, n, a, W, de, ld, bw);
+}
+
 // wyb (FP32 only, may be null): run the back-transformation as blocked
 // reflectors on the matrix cores (the apply kernel then only replays the QL
 // rotations from the identity) in a region of WyLayout(chunk, n, 4) bytes.
@@ -620,14 +638,7 @@ hipError_t launch_split_large(int L, int nm, int n, T *a, T *w, int *info, int s
       unsigned grid = tg;
       if (gc) grid = (unsigned)(128 * gc) < grid ? (unsigned)(128 * gc) : grid;
       if (sym && tc == 0) {
-        // register-resident: 12 waves own the <= 36 tiles of n <= 256 (one
-        // workgroup per CU), 4 waves the <= 10 tiles of n <= 128
-        if (n <= 128)
-          hipLaunchKernelGGL((eig_tri_reg_kernel<T, 4, 3, 3>), dim3(grid), dim3(256), 0, s, cur, nm, n, ac, Wm, de,
-                             lc, bw);
-        else
-          hipLaunchKernelGGL((eig_tri_reg_kernel<T, 12, 3, 3>), dim3(grid), dim3(768), 0, s, cur, nm, n, ac, Wm, de,
-                             lc, bw);
+        launch_tri_reg<T>(L, cur, nm, n, ac, Wm, de, lc, bw, grid, s);
       } else if (sym) {
         if (cfg == 3)
           hipLaunchKernelGGL((eig_tri_large_kernel<T, 1024, TriNbp<T>::value, 256, 4, true>), dim3(grid), dim3(1024), 0, s, cur,
@@ -997,7 +1008,6 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
   int *st = (int *)(base + lay.st);
   const int ph = (solver & FLAG_PH_ALL) ? (solver & FLAG_PH_ALL) : FLAG_PH_ALL;
   if (ph != FLAG_PH_ALL && L > lc) return hipErrorInvalidValue;
-  const bool xq = dc_explicit_q(L, n, tb);
   const int nanfail = L < (tb == 4 && n <= 128 ? SPLIT_MIN_L : SPLIT_LARGE_MIN_L) ? 1 : 0;
   const int nblk = (n + 63) / 64, nb16 = (n + 15) / 16, mcols = n - kopt_mdrop(kop);
   DcNodes lev[4] = {};
@@ -1010,16 +1020,8 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
     int *ic = info ? info + c0 : nullptr;
     const unsigned tg = (unsigned)(cur < 1024 ? cur : 1024);
     if (ph & FLAG_PH_TRI) {
-      if (xq) {
-        if constexpr (tb == 4)
-          hipLaunchKernelGGL((eig_tri_kernel<T, 128>), dim3((unsigned)cur), dim3(128), 0, s, cur, nm, n, (const T *)ac,
-                             Wm, de, lc, UvSplitArgs{}, (const int *)nullptr);
-      } else if (n <= 128) {
-        hipLaunchKernelGGL((eig_tri_reg_kernel<T, 4, 3, 3>), dim3(tg), dim3(256), 0, s, cur, nm, n, (const T *)ac, Wm,
-                           de, lc, bw);
-      } else if (n <= 256) {
-        hipLaunchKernelGGL((eig_tri_reg_kernel<T, 12, 3, 3>), dim3(tg), dim3(768), 0, s, cur, nm, n, (const T *)ac,
-                           Wm, de, lc, bw);
+      if (n <= 256) {
+        launch_tri_reg<T>(L, cur, nm, n, (const T *)ac, Wm, de, lc, bw, tg, s);
       } else {
         // the strips in the first buffer of vectors, which is free until the merges
         constexpr int NBP = tb == 8 ? 8 : 16, NT = tb == 8 ? 512 : 1024;
@@ -1056,25 +1058,14 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
       }
     }
     if (ph & FLAG_PH_APPLY) {
-      if (xq) {
-        GemmArgs g{};
-        const long long nn = (long long)n * n;
-        g.M = n; g.N = mcols; g.K = n; g.batch = cur; g.alpha = 1.0; g.skip = st;
-        g.A = Wm; g.lda = n; g.sa = nn;
-        g.B = Z[0]; g.ldb = n; g.sb = nn;
-        g.C = ac; g.ldc = nm; g.sc = (long long)nm * n;
-        const hipError_t err = gemm_launch(KIND, g, s);
-        if (err != hipSuccess) return err;
-      } else {
-        const long long blocks = (long long)cur * nb16;
-        hipLaunchKernelGGL((eig_dc_wyt_kernel<T>), dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, blocks, n,
-                           nb16, (const T *)Wm, (const T *)bw, U);
-        constexpr int W8 = tb == 8 ? 3 : 4, W16 = tb == 8 ? 2 : 3, W24 = tb == 8 ? 2 : 3, W32 = tb == 8 ? 1 : 2;
-        if (n <= 128) launch_dc_back<T, 8, W8>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
-        else if (n <= 256) launch_dc_back<T, 16, W16>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
-        else if (n <= 384) launch_dc_back<T, 24, W24>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
-        else launch_dc_back<T, 32, W32>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
-      }
+      const long long blocks = (long long)cur * nb16;
+      hipLaunchKernelGGL((eig_dc_wyt_kernel<T>), dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, blocks, n,
+                         nb16, (const T *)Wm, (const T *)bw, U);
+      constexpr int W8 = tb == 8 ? 3 : 4, W16 = tb == 8 ? 2 : 3, W24 = tb == 8 ? 2 : 3, W32 = tb == 8 ? 1 : 2;
+      if (n <= 128) launch_dc_back<T, 8, W8>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+      else if (n <= 256) launch_dc_back<T, 16, W16>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+      else if (n <= 384) launch_dc_back<T, 24, W24>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
+      else launch_dc_back<T, 32, W32>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
     }
   }
   return hipGetLastError();
@@ -1893,7 +1884,8 @@ hipError_t launch_params(int L, int n, int tb, int solver, int *p)
     grp(nb_of(n), L < lchunk(solver) ? L : lchunk(solver), 64);
   } else if (use_dc_large(L, n, tb, solver)) {
     const int lc = L < lchunk_large(solver) ? L : lchunk_large(solver);
-    if (dc_explicit_q(L, n, tb)) {
+    // callers are told the shapes they always were: order class and matrices in flight
+    if (tb == 4 && n <= 128 && L >= SPLIT_MIN_L) {
       grp(128, lc, 128);
     } else {
       p[0] = 256; p[1] = lc < 1024 ? lc : 1024; p[2] = 1; p[3] = 256;

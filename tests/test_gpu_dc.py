@@ -86,6 +86,21 @@ def test_families_of_several_blocks(n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [65, 128, 129, 160, 191, 192, 193])
+def test_families_in_large_batches(n, dtype):
+    """More than 256 matrices (128 < n <= 192: the three-block tridiagonalisation)."""
+    print(f"[dc] n={n} {np.dtype(dtype).name}", flush=True)
+    f = families(n, np.random.default_rng(n)).astype(dtype)
+    t = torch.from_numpy(np.tril(f)).repeat(17, 1, 1).to(DEV)
+    z, w, info = eg.eigen_batch(t, path="dc")
+    torch.cuda.synchronize()
+    assert int(info.abs().max()) == 0
+    z, w = z.view(17, *f.shape), w.view(17, *f.shape[:2])
+    assert torch.equal(z, z[:1].expand_as(z)) and torch.equal(w, w[:1].expand_as(w))
+    check(f, z[0].cpu().numpy(), w[0].cpu().numpy(), dtype)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n", [257, 264, 272])
 def test_more_matrices_than_workgroups(n, dtype):
     """Above 1024 matrices a workgroup of the tridiagonalisation takes a second one:
