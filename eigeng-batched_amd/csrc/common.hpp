@@ -102,6 +102,13 @@ __device__ __forceinline__ T lane_bcast(T x, int src)
   return lane_move(x, [addr](int v) { return __builtin_amdgcn_ds_bpermute(addr, v); });
 }
 
+// The same for a source that is uniform over the wave, without the LDS crossbar.
+template <typename T>
+__device__ __forceinline__ T lane_read(T x, int src)
+{
+  return lane_move(x, [src](int v) { return __builtin_amdgcn_readlane(v, src); });
+}
+
 // Ballot restricted to this lane's group, shifted so bit 0 is the group's lane 0.
 template <int NB>
 __device__ __forceinline__ uint64_t group_ballot(bool p)

@@ -19,6 +19,7 @@
 #include "eig_split_large.hpp"
 #include "eig_tri_reg.hpp"
 #include "eig_tri_stream.hpp"
+#include "eig_tri_wave.hpp"
 #include "eig_dc.hpp"
 #include "eig_dc_large.hpp"
 #include "eig_check.hpp"
@@ -411,13 +412,25 @@ hipError_t launch_split(int L, int nm, int n, T *a, T *w, int *info, int solver,
 // DcLayout.  Phases: tridiagonalisation with Q; the second one nothing; merges and
 // store.  nanfail, only: see eig_dc_kernel.
 template <typename T, int NB, int NBT, int NLR>
-void launch_dc_chunk(int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, int nanfail, T *q, T *de, int ld,
-                     const int *only, hipStream_t s)
+void launch_dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, int nanfail, T *q, T *de,
+                     int ld, const int *only, hipStream_t s)
 {
   constexpr int G = GroupShape<NBT>::G;
-  if (ph & FLAG_PH_TRI)
-    hipLaunchKernelGGL((eig_tri_kernel<T, NBT>), dim3((unsigned)((cur + G - 1) / G)), dim3(64), 0, s, cur, nm, n, a, q,
-                       de, ld, UvSplitArgs{}, only);
+  if (ph & FLAG_PH_TRI) {
+    // One matrix per wave for n > 32 (eig_tri_wave.hpp).  For 16 < n <= 32 its chain is
+    // shorter, but two matrices in a wave are less work once the chip is full (n = 32,
+    // L = 1024, 2048, 4096: FP32 24, 34, 59 us against 39, 43, 51; FP64 33, 51, 83
+    // against 45, 54, 72).  By L, not by the chunk: a divided batch gives the same bits.
+    constexpr int NS = NB / 16, WPE = sizeof(T) == 4 ? 4 : (NS == 2 ? 3 : 2);
+    if (NS > 2 || (NS == 2 && L <= 2048)) {
+      if constexpr (NS >= 2)
+        hipLaunchKernelGGL((eig_tri_wave_kernel<T, NS, WPE>), dim3((unsigned)cur), dim3(64), 0, s, cur, nm, n,
+                           (const T *)a, q, de, ld, only);
+    } else if constexpr (NS <= 2) {
+      hipLaunchKernelGGL((eig_tri_kernel<T, NBT>), dim3((unsigned)((cur + G - 1) / G)), dim3(64), 0, s, cur, nm, n, a,
+                         q, de, ld, UvSplitArgs{}, only);
+    }
+  }
   if (ph & FLAG_PH_APPLY)
     hipLaunchKernelGGL((eig_dc_kernel<T, NB, NLR, false>), dim3((unsigned)cur), dim3(NB * NLR), 0, s, cur, nm, n, a,
                        (const T *)q, (const T *)de, ld, w, info, kop, nanfail, 1, (T *)nullptr, (T *)nullptr, 0, only);
@@ -427,7 +440,7 @@ void dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int 
               const int *only, hipStream_t s)
 {
   const int nanfail = L < split_min_l(n, (int)sizeof(T)) ? 1 : 0;
-#define DC(NB, NBT, NLR) launch_dc_chunk<T, NB, NBT, NLR>(cur, nm, n, a, w, info, ph, kop, nanfail, q, de, ld, only, s)
+#define DC(NB, NBT, NLR) launch_dc_chunk<T, NB, NBT, NLR>(L, cur, nm, n, a, w, info, ph, kop, nanfail, q, de, ld, only, s)
   if (n <= 8) DC(16, 8, 4);
   else if (n <= 16) DC(16, 16, 4);
   // one wave a matrix does fewer instructions, two have the shorter chain
