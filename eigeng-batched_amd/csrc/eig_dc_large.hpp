@@ -315,24 +315,31 @@ __global__ __launch_bounds__(256) void eig_dc_wyt_kernel(long long blocks, int n
 
 // V: columns of Zs (ld n), 16 per wave, all NT row tiles in registers; per block
 // of reflectors P = U^T V (rows up to the block), P <- T P, V <- V + U P, the
-// accumulator layout of one product being the operand layout of the next.  The
-// reflectors come from L2 in 64-row groups, every load of a group issued before
-// its products.  Loads are not clamped to the matrix: they stay within the
-// workspace (16 NT - n rows past a column, 15 columns past the last), whose
-// regions of eigenvectors follow W's, and what lies outside u_c is replaced by
-// zero.  Result to a (ld nm, columns below mcols).
+// accumulator layout of one product being the operand layout of the next.  The four
+// waves of a workgroup share the block through LDS (columns below the diagonal as
+// they are, zeros elsewhere), the next block's loads in flight meanwhile; a column
+// has BS elements there, which puts the 16 columns of an operand on different banks.
+// Loads are not clamped to the matrix: they stay within the workspace (16 NT - n
+// rows past a column, 15 columns past the last), whose regions of eigenvectors
+// follow W's, and what lies outside u_c is replaced by zero.  Result to a (ld nm,
+// columns below mcols).
+// What bounds it: the matrix cores wait for one LDS operand per instruction (n = 256 in
+// FP64: 4 n^3 operations are 3.8 of 8192 matrices' 7.1 ms).  With every wave reading the
+// reflectors for itself, twice, from L2, the whole back-transformation took 14.6 ms, now
+// 8.2; n = 128 in FP32 1.14 and 0.88; 64 matrices of n = 512 in FP64 1.00 and 0.58.
 template <typename T, int NT, int WPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void eig_dc_back_kernel(
     int cur, int n, int nm, int mcols, int ncg, const T *__restrict__ W, const T *__restrict__ Tm,
     const T *__restrict__ Zs, T *__restrict__ a, const int *__restrict__ st)
 {
   typedef typename Mfma16<T>::v4 v4;
-  constexpr int NG = NT / 4;
+  constexpr int NR = 16 * NT, BS = NR + (sizeof(T) == 8 ? 2 : 4);
+  __shared__ T Ub[16 * BS];
   const long long total = (long long)cur * ncg, lid = gemm_xcd_remap(blockIdx.x, total);
   const int mat = (int)(lid / ncg), cg = (int)(lid - (long long)mat * ncg);
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, m = lane & 15, g = lane >> 4;
+  if (st[mat] != 0) return;                                 // the whole workgroup
   const int col = 64 * cg + 16 * wv + m;
-  if (64 * cg + 16 * wv >= mcols || st[mat] != 0) return;   // the whole wave
   const int nb16 = (n + 15) >> 4;
   const T *__restrict__ Wm = W + (size_t)mat * n * n;
   const T *__restrict__ Zm = Zs + (size_t)mat * n * n + (size_t)(col < n ? col : n - 1) * n;
@@ -345,64 +352,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
       const T x = Zm[k];
       V[t][r] = (k < n) ? x : T(0);
     }
+  // thread t of the workgroup: rows (t & 63) + 64 i of the columns (t >> 6) + 4 j
+  constexpr int NI = NR / 64;
+  T x[NI][4];
+  auto load = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (4 * i <= b) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[i][j] = Wm[(size_t)(16 * b + (tid >> 6) + 4 * j) * n + (tid & 63) + 64 * i];
+      }
+  };
+  load(0);
 #pragma unroll 1
   for (int b = 0; b < nb16; ++b) {
-    const int c0 = 16 * b;
-    // u_{c0+m} as rows of U^T
-    const int c = c0 + m;
-    const T *__restrict__ uc = Wm + (size_t)(c < n ? c : n - 1) * n;
-    const int lim = c < n ? c : 0;
+    __syncthreads();                                        // the block before is used up
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (4 * i <= b) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c = 16 * b + (tid >> 6) + 4 * j, k = (tid & 63) + 64 * i;
+          Ub[((tid >> 6) + 4 * j) * BS + k] = (k < c && c < n) ? x[i][j] : T(0);
+        }
+      }
+    const T *__restrict__ tp = Tm + ((size_t)mat * nb16 + b) * 256 + 4 * lane;
+    T ta[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ta[r] = tp[r];
+    __syncthreads();
+    load(b + 1 < nb16 ? b + 1 : b);
     v4 P0 = v4{0, 0, 0, 0}, P1 = v4{0, 0, 0, 0};
 #pragma unroll
-    for (int G = 0; G < NG; ++G) {
+    for (int G = 0; G < NT / 4; ++G) {
       if (4 * G <= b) {
-        T x[4][4];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int k = 16 * (4 * G + tt) + Mfma16<T>::row(g, r);
-            x[tt][r] = uc[k];
-          }
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int k = 16 * (4 * G + tt) + Mfma16<T>::row(g, r);
-            const T y = (k < lim) ? x[tt][r] : T(0);
+            const T y = Ub[m * BS + 16 * (4 * G + tt) + Mfma16<T>::row(g, r)];
             if (tt & 1) P1 = Mfma16<T>::op(y, V[4 * G + tt][r], P1);
             else P0 = Mfma16<T>::op(y, V[4 * G + tt][r], P0);
           }
       }
     }
-    const T *__restrict__ tp = Tm + ((size_t)mat * nb16 + b) * 256 + 4 * lane;
     v4 Q = v4{0, 0, 0, 0};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Q = Mfma16<T>::op(tp[r], P0[r] + P1[r], Q);
-    // columns c0 + row(g, r) of U as rows
-    const T *__restrict__ ur[4];
-    int lr[4];
+    for (int r = 0; r < 4; ++r) Q = Mfma16<T>::op(ta[r], P0[r] + P1[r], Q);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int cr = c0 + Mfma16<T>::row(g, r);
-      ur[r] = Wm + (size_t)cr * n + m;
-      lr[r] = (cr < n ? cr : 0) - m;                        // rows 16 t + m below cr: 16 t < lr
-    }
-#pragma unroll
-    for (int G = 0; G < NG; ++G) {
+    for (int G = 0; G < NT / 4; ++G) {
       if (4 * G <= b) {
-        T x[4][4];
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) x[tt][r] = ur[r][16 * (4 * G + tt)];
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const T y = (16 * (4 * G + tt) < lr[r]) ? x[tt][r] : T(0);
-            V[4 * G + tt] = Mfma16<T>::op(y, Q[r], V[4 * G + tt]);
-          }
+          for (int r = 0; r < 4; ++r)
+            V[4 * G + tt] = Mfma16<T>::op(Ub[Mfma16<T>::row(g, r) * BS + 16 * (4 * G + tt) + m], Q[r], V[4 * G + tt]);
       }
     }
   }
