@@ -196,21 +196,21 @@ bool use_split128(int L, int n, int tbytes, int solver)
 // choice of the caller's (chunk and phase bits aside), 8 <= n <= 64.  Measured on
 // one MI355X, random symmetric matrices, against the better of the fused and the
 // split path (us, that / divide and conquer): L = 64: n = 8 42 / 23 (FP32), 50 / 29
-// (FP64); n = 16 104 / 28, 132 / 40; n = 32 277 / 60, 363 / 75; n = 64 819 / 157,
-// 1094 / 188.  L = 2048: n = 8 44 / 25, 54 / 37; n = 16 110 / 38, 145 / 56; n = 32
-// 300 / 85, 399 / 121; n = 64 912 / 263, 1393 / 452.  On large batches the QL
-// recurrence's latency is shared by more matrices, and orders that fill their
+// (FP64); n = 16 104 / 28, 132 / 40; n = 32 277 / 48, 363 / 61; n = 64 819 / 103,
+// 1094 / 132.  L = 2048: n = 8 44 / 25, 54 / 37; n = 16 110 / 38, 145 / 56; n = 32
+// 300 / 76, 399 / 117; n = 64 912 / 235, 1393 / 373.  On large batches the QL
+// recurrence's latency is shared by more matrices, and small orders that fill their
 // padded tiles badly lose: L = 16384: n = 8 52 / 67, 78 / 142; n = 9 80 / 86,
 // 101 / 175; n = 12 103 / 90, 146 / 189; n = 20 258 / 213, 385 / 443; n = 33
-// 784 / 667, 1372 / 1489; n = 40 990 / 764, 1802 / 1690; n = 64 1915 / 1364,
-// 3742 / 3190; those keep the QL paths from about where the two lines cross.
+// 791 / 616, 1380 / 1326; n = 40 990 / 654, 1782 / 1432; n = 64 1891 / 1098,
+// 3618 / 2543; those keep the QL paths from about where the two lines cross.
 constexpr int DC_MIN_N = 8;
 int dc_max_l(int n, int tbytes)
 {
   if (n <= 8) return 4096;
   if (tbytes == 4) return n <= 10 ? 12288 : 0x7fffffff;
   if (n <= 16) return 6144;
-  return (n <= 23) ? 8192 : (n >= 33 && n <= 37) ? 12288 : 0x7fffffff;
+  return n <= 23 ? 8192 : 0x7fffffff;
 }
 // FLAG_SPLIT asks for the path in separate kernels: on batches that take it by
 // themselves that is this one, smaller ones get the QL recurrence.
@@ -233,7 +233,7 @@ bool use_dc_large(int L, int n, int tbytes, int solver)
   return (flags & FLAG_DC) || !(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L;
 }
 
-// Its workspace for a chunk of lc matrices: the reflectors (or Q), d / e, beta, two
+// Its workspace for a chunk of lc matrices: the reflectors, d / e, beta, two
 // buffers of eigenvectors of T, the merges' U (later the reflector blocks' T), status.
 struct DcLargeLayout {
   size_t wm, de, bw, z0, z1, u, st, total;
