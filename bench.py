@@ -149,12 +149,13 @@ def tuned_line(a0, plain_ms, steps, warmup):
 
 
 def time_phases(a0, steps, warmup, path="split"):
-    """Per-phase HIP-event times (ms) of the split paths: the phases are issued
-    as separate library calls on one stream with events between them (n <= 64:
-    tri = eig_tri_kernel, ql = eig_ql_reg_kernel, apply = eig_apply_kernel plus
-    the overflow-fallback launch; larger n: eig_tri_reg_kernel (n <= 256),
-    eig_ql_lane_kernel, eig_apply_large_kernel plus the fallback launch, whose
-    workgroups exit at once when no matrix overflowed).  Returns {phase: mean ms}."""
+    """Per-phase HIP-event times (ms) of a path in separate kernels: the phases are
+    issued as separate library calls on one stream with events between them.  For
+    batches that take divide and conquer (from 2048 matrices) with n <= 64: tri =
+    eig_tri_wave_kernel (eig_tri_kernel for n <= 32), ql = nothing, apply =
+    eig_dc_kernel; larger n: tri = eig_tri_reg_kernel (n <= 256) or
+    eig_tri_stream_kernel, ql = the merges, apply = the back-transformation.
+    Returns {phase: mean ms}."""
     import numpy as np
     import torch
     import eigeng_batched as eg
@@ -327,7 +328,7 @@ def bench_n32(steps, warmup, tuned=True):
             "launch": {k: p[k] for k in ("grpSZ", "numTB", "numGR", "numTH")},
             "roofline": {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                          "frac": gbs / PEAK_HBM_GBS, "bytes_per_matrix": b,
-                         "kernel": "split path: eig_tri_kernel<double,32> + eig_ql_reg_kernel + eig_apply_kernel",
+                         "kernel": "eig_tri_wave_kernel<double,2> + eig_dc_kernel<double,32>",
                          "valu_tflops": tfs, "valu_frac_fp64": tfs / PEAK_FP64_TFLOPS},
             "tuned": tl}
 
@@ -528,13 +529,13 @@ def bench_n256(steps, warmup, vendor=True, tuned=True, mixed=True):
             "roofline": {"bound": "valu", "achieved": L2 * f2 / (kms2 * 1e-3) / 1e12,
                          "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                          "frac": L2 * f2 / (kms2 * 1e-3) / 1e12 / PEAK_FP64_TFLOPS,
-                         "kernel": "eig_tri_reg_kernel + eig_ql_lane_kernel + eig_apply_large_kernel "
-                                   "(+ overflow-fallback launch)",
+                         "kernel": "eig_tri_reg_kernel + eig_dc_kernel + eig_dc_merge_kernel + eig_dc_update_kernel + "
+                                   "eig_dc_wyt_kernel + eig_dc_back_kernel",
                          "kernel_ms": kms2, "phase_ms": ph2,
                          "note": "(10/3)n^3 flops per matrix against the FP64 vector peak"},
             "roofline_hbm": {"achieved": L2 * b2 / (kms2 * 1e-3) / 1e9, "peak": PEAK_HBM_GBS,
                              "unit": "GB/s", "bytes_per_matrix": b2,
-                             "traffic": _traffic("traffic_eig_split_n256_fp64.json")}}
+                             "traffic": _traffic("traffic_eig_dc_n256_fp64.json")}}
 
 
 def gemm_f64_roofline(batch, n, reps=5):
@@ -716,9 +717,8 @@ def chunk_tradeoff(a0, shifts, steps=5, warmup=1):
 
 
 def bench_n128(steps, warmup):
-    """L = 8192, n = 128, FP32 line (the register split path, the default for
-    FP32 64 < n <= 128 from 2048 matrices): whole-call time, per-phase times,
-    roofline, accuracy of every matrix."""
+    """L = 8192, n = 128, FP32 line: whole-call time, per-phase times, roofline,
+    accuracy of every matrix."""
     import torch
     L2, n2 = 8192, 128
     q0 = make_qdq_gpu(L2, n2, seed=0xE16E0005, dtype=torch.float32)
@@ -727,7 +727,7 @@ def bench_n128(steps, warmup):
     bad = int((info2 != 0).sum().item())
     del a2, w2
     torch.cuda.empty_cache()
-    ph2, a2, w2, _ = time_phases(q0, 2, 1, path="split-reg128")
+    ph2, a2, w2, _ = time_phases(q0, 2, 1)
     del q0, a2, w2
     torch.cuda.empty_cache()
     kms2 = sum(ph2.values())
@@ -739,13 +739,13 @@ def bench_n128(steps, warmup):
             "roofline": {"bound": "valu", "achieved": L2 * f2 / (kms2 * 1e-3) / 1e12,
                          "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                          "frac": L2 * f2 / (kms2 * 1e-3) / 1e12 / PEAK_FP32_TFLOPS,
-                         "kernel": "eig_tri_kernel<float,128> + eig_ql_reg_kernel<float,128> + eig_apply_kernel<float,128> "
-                                   "(+ overflow-fallback launch)",
+                         "kernel": "eig_tri_reg_kernel + eig_dc_kernel + eig_dc_merge_kernel + eig_dc_update_kernel + "
+                                   "eig_dc_wyt_kernel + eig_dc_back_kernel",
                          "kernel_ms": kms2, "phase_ms": ph2,
                          "note": "(10/3)n^3 flops per matrix against the FP32 vector peak"},
             "roofline_hbm": {"achieved": L2 * b2 / (kms2 * 1e-3) / 1e9, "peak": PEAK_HBM_GBS,
                              "unit": "GB/s", "bytes_per_matrix": b2,
-                             "traffic": _traffic("traffic_eig_split128_n128_fp32.json")}}
+                             "traffic": _traffic("traffic_eig_dc_n128_fp32.json")}}
 
 
 def host_threads():
@@ -923,16 +923,16 @@ def main():
     peak_c = PEAK_FP32_TFLOPS if args.dtype == "fp32" else PEAK_FP64_TFLOPS
     if phases:
         # the step is a sequence of kernels: the roof is taken over their summed
-        # event-timed durations (the fallback launch included in "apply")
+        # event-timed durations
         kern_ms = sum(phases.values())
-        kernel = "eig_tri_kernel + eig_ql_reg_kernel + eig_apply_kernel (+ overflow-fallback launch)"
+        kernel = "eig_tri_wave_kernel + eig_dc_kernel"
     else:
         kern_ms = ms
         kernel = "one solver kernel per step"
     achieved_tf = L * flops / (kern_ms * 1e-3) / 1e12
     achieved_gbs = L * bytes_alg / (kern_ms * 1e-3) / 1e9
     traffic = None
-    tfile = os.path.join(ROOT, "profiles", f"traffic_eig_{'split' if phases else 'wave'}_n{n}_{args.dtype}.json")
+    tfile = os.path.join(ROOT, "profiles", f"traffic_eig_{'dc' if phases else 'wave'}_n{n}_{args.dtype}.json")
     if os.path.exists(tfile):
         with open(tfile) as f:
             traffic = json.load(f).get("bytes_per_launch")
@@ -958,8 +958,8 @@ def main():
                      "frac": achieved_tf / peak_c, "traffic": traffic, "kernel": kernel,
                      "kernel_ms": kern_ms, "phase_ms": phases,
                      "note": "compute roof at the reference's (10/3)n^3 flops per matrix over the "
-                             "event-timed kernel time; the kernels run on the VALU (no MFMA), so "
-                             "the peak is the FP vector peak"},
+                             "event-timed kernel time against the FP vector peak, where most of "
+                             "the work runs (Q and the merges' products run on MFMA)"},
         "roofline_hbm": {"achieved": achieved_gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                          "frac": achieved_gbs / PEAK_HBM_GBS, "bytes_per_matrix": bytes_alg},
         "wall_s_including_restores": wall,
