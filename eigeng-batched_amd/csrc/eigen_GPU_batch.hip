@@ -136,7 +136,7 @@ struct SplitLargeLayout {
 };
 
 // Smallest batch for which the split path (tridiagonalisation, lane-per-matrix
-// QL, replay) is the default for n <= 64 rather than the fused one-kernel
+// QL, replay) is the QL path for n <= 64 rather than the fused one-kernel
 // path.  Measured on one MI355X, random symmetric matrices, L = 128..2048
 // (split / fused ms): FP64 n = 16..32 the split path wins at every batch size
 // (n = 32: 0.36 / 0.42 at L = 128, 0.38 / 0.48 at L = 1024; n = 20 within 2 %
@@ -179,7 +179,7 @@ bool use_split_large(int L, int n, int tbytes, int solver)
   return L >= (use_wave_kernel(n, tbytes) ? SPLIT_MIN_L : SPLIT_LARGE_MIN_L);
 }
 
-// FP32 64 < n <= 128: the register split path is the default from
+// FP32 64 < n <= 128: the register split path is the QL path from
 // SPLIT_MIN_L matrices on (measured at L = 8192: n = 128 12.3 ms, against
 // 24.2 ms for the large-order split path and 59 ms for the fused kernel);
 // FLAG_SPLIT still selects the large-order split path

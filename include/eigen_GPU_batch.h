@@ -54,7 +54,10 @@ void eigen_GPU_batch_FP(const int L, const int nm, const int n, const int m,
 
 /* Solver selection for the _x entry points. */
 enum eigen_GPU_batch_solver {
-  EIGEN_GPU_BATCH_IMTQL2 = 0, /* Householder + implicit-shift QL + back-transform (default) */
+  /* the default: Householder, the tridiagonal eigenproblem, back-transform; the middle step by
+   * divide and conquer, or implicit-shift QL for shapes where that is faster, the unsorted
+   * order and the path bits below */
+  EIGEN_GPU_BATCH_IMTQL2 = 0,
   EIGEN_GPU_BATCH_TQL2 = 1,   /* Householder + explicit-shift QL (the reference's shipped QL) */
   EIGEN_GPU_BATCH_JACOBI = 2, /* two-sided Jacobi on the full matrix (jac_tiled.hpp) */
   /* FP64 entry points only, n <= 256: mixed precision.  The matrices rounded to
@@ -81,19 +84,24 @@ enum eigen_GPU_batch_solver {
 
 /*
  * Tuning bits OR-ed into `solver` of the _x entry points and of
- * eigen_GPU_batch_bufsize (the default picks by n, precision and L: for n <= 64
- * the split path from 2048 matrices, from one matrix for FP64 16 <= n <= 32 and
- * FP32 28 <= n <= 32, from 1024 for FP32 n >= 56, the fused kernel below):
+ * eigen_GPU_batch_bufsize.  The default picks by n, precision and L: with IMTQL2
+ * divide and conquer for n >= 8, except large batches of small orders (n = 8 above
+ * 4096 matrices, FP32 n <= 10 above 12288, FP64 n <= 16 above 6144 and n <= 23 above
+ * 8192); otherwise QL, for n <= 64 the split path from 2048 matrices, from one matrix
+ * for FP64 16 <= n <= 32 and FP32 28 <= n <= 32, from 1024 for FP32 n >= 56, the
+ * fused kernel below:
  *   0x100  one fused kernel per matrix group;
- *   0x200  split n <= 64 path: register tridiagonalisation, one-lane-per-matrix
- *          QL recurrence writing a rotation log, rotation apply kernel;
+ *   0x200  separate kernels: divide and conquer from 2048 matrices, below that the
+ *          split path (register tridiagonalisation, one-lane-per-matrix QL
+ *          recurrence writing a rotation log, rotation apply kernel);
+ *   0x8000000 (IMTQL2) divide and conquer whatever the shape, n <= 512;
  *   0x400  (with 0x200) shrink the rotation log so every matrix takes the
  *          split path's overflow fallback (a host-forced test of that path);
- *   0x1000 / 0x2000 / 0x4000  run only the split path's tridiagonalisation /
- *          QL / apply phase (L <= 16384): successive calls on one stream with
+ *   0x1000 / 0x2000 / 0x4000  run only the tridiagonalisation / QL (or merges) /
+ *          apply phase of a path in separate kernels (L <= 16384): successive calls on one stream with
  *          one workspace compose the full solve, so each phase can be timed;
  *   0x8000 FP32 64 < n <= 128: the register split path (two-wave
- *          tridiagonalisation, lane-per-matrix QL, 64-row-block apply), the
+ *          tridiagonalisation, lane-per-matrix QL, 64-row-block apply), TQL2's
  *          default there from 2048 matrices; 0x200 selects the large-order
  *          split path instead;
  *   bits 16-17 / 20-23  workgroup size / resident workgroup count of the
