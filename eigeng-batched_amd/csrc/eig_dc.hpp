@@ -28,6 +28,9 @@
 //      working precision without extended arithmetic.
 //   4. the new eigenvalues are ranked, the vectors U formed in that order, and
 //      Q <- Q U on the matrix cores.
+// Steps 1-3 run on the node scaled by a power of two to a largest entry of order one,
+// whatever its size against the rest of T: the products of step 3 hold one factor of
+// (node's size) / HUGE_, and the derivative in step 2 is of the order of 1 / size.
 #pragma once
 #include "common.hpp"
 #include "eig_symdmt.hpp"
@@ -35,7 +38,7 @@
 
 namespace eigmi {
 
-// HUGE_ (T is scaled to a largest entry of order one): from here on a value
+// HUGE_ (a node is scaled to a largest entry of order one): from here on a value
 // stands for "no pole"; slot p of a node uses HUGE_ (1 + p / 1024), so that
 // these sort behind the poles in the order of their slots.  STEP: 4 sqrt(eps).
 template <typename T> struct DcLim;
@@ -459,9 +462,9 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
   const int end = (base + S < n) ? base + S : n;               // live columns of the node end here
   const bool both = mid < n;                                   // the node has a right child
   // ---- 1. z, the poles set aside, ranks --------------------------------------
-  T z = T(0), rho = T(0), key = HUGE_, dmax = T(0);
+  T z = T(0), rho = T(0), key = HUGE_, dmax = T(0), sc = T(1);
   bool nd = false;
-  int c = 0, k = 0;
+  int c = 0, k = 0, ex = 0;
   if (on) {
     const T er = both ? Sh.e[mid - 1] : T(0);
     const T di = Sh.d[i];
@@ -473,8 +476,14 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
       dmax = max_(dmax, max_(abs_(Sh.d[base]), abs_(Sh.d[(both ? mid : end) - 1])));
       if (both) dmax = max_(dmax, max_(abs_(Sh.d[mid]), abs_(Sh.d[end - 1])));
     }
+    // steps 1-3 on the node scaled to order one (a power of two: exact)
+    if (dmax > T(0)) (void)frexp(dmax, &ex);
+    ex = max(min(ex, DcLim<T>::EXP), -DcLim<T>::EXP);
+    sc = ldexp(T(1), -ex);
+    rho *= sc;
+    dmax *= sc;
     nd = i < n && rho * abs_(z) > T(2) * eps * dmax;
-    key = nd ? di : HUGE_ * (T(1) + T(p) * T(1.0 / 1024));
+    key = nd ? di * sc : HUGE_ * (T(1) + T(p) * T(1.0 / 1024));
     if (sub == 0) Sh.key[i] = key;
   }
   dc_sync<LW>();
@@ -547,7 +556,11 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
     dc_root<T, S, LN, REG>(&Sh.dl[base], &Sh.zq[base], k, p, sub, rho, root, a0, t0);
     if (root) { da = a0; tau = t0; }
     s0 = Sh.src[i] & 63;
-    v0 = root ? da + tau : Sh.d[s0];
+    if (s0 >= n) {                                             // no column: HUGE_ in every scale
+      sc = T(1);
+      ex = 0;
+    }
+    v0 = root ? da + tau : Sh.d[s0] * sc;
     if (sub == 0) {
       Sh.da[i] = da;
       Sh.tau[i] = tau;
@@ -581,7 +594,7 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
       Sh.ma[nr] = da;
       Sh.mt[nr] = tau;
       Sh.mdef[nr] = root ? -1 : s0;
-      Sh.d[nr] = v0;          // every read of the old values is before the last barrier
+      Sh.d[nr] = ldexp(v0, ex);   // every read of the old values is before the last barrier
     }
   }
   dc_sync<NW>();
