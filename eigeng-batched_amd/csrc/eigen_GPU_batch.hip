@@ -436,10 +436,9 @@ void launch_dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int p
                        (const T *)q, (const T *)de, ld, w, info, kop, nanfail, 1, (T *)nullptr, (T *)nullptr, 0, only);
 }
 template <typename T>
-void dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, T *q, T *de, int ld,
-              const int *only, hipStream_t s)
+void dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, int nanfail, T *q, T *de,
+              int ld, const int *only, hipStream_t s)
 {
-  const int nanfail = L < split_min_l(n, (int)sizeof(T)) ? 1 : 0;
 #define DC(NB, NBT, NLR) launch_dc_chunk<T, NB, NBT, NLR>(L, cur, nm, n, a, w, info, ph, kop, nanfail, q, de, ld, only, s)
   if (n <= 8) DC(16, 8, 4);
   else if (n <= 16) DC(16, 16, 4);
@@ -461,10 +460,11 @@ hipError_t run_dc(int L, int nm, int n, T *a, T *w, int *info, int solver, int k
   T *q = (T *)(base + lay.q), *de = (T *)(base + lay.de);
   const int ph = (solver & FLAG_PH_ALL) ? (solver & FLAG_PH_ALL) : FLAG_PH_ALL;
   if (ph != FLAG_PH_ALL && L > lc) return hipErrorInvalidValue;
+  const int nanfail = L < split_min_l(n, (int)sizeof(T)) ? 1 : 0;
   for (long long c0 = 0; c0 < L; c0 += lc) {
     const int cur = (int)((L - c0) < lc ? (L - c0) : lc);
-    dc_chunk<T>(L, cur, nm, n, a + (size_t)c0 * nm * n, w + (size_t)c0 * n, info ? info + c0 : nullptr, ph, kop, q, de,
-                lc, nullptr, s);
+    dc_chunk<T>(L, cur, nm, n, a + (size_t)c0 * nm * n, w + (size_t)c0 * n, info ? info + c0 : nullptr, ph, kop,
+                nanfail, q, de, lc, nullptr, s);
   }
   return hipGetLastError();
 }
@@ -1575,9 +1575,10 @@ hipError_t run_warm(int L, int nm, int n, int m, T *a, const T *q0, T *w, void *
     hipLaunchKernelGGL((eig_warm_store_kernel<T>), dim3((unsigned)(cur < 16384 ? cur : 16384)), dim3(256), 0, s, cur,
                        nm, n, m, (const T *)v, (const int *)ji, st, ac, ic);
     // the matrices left over: the path a plain call of this batch takes (small
-    // batches' when that is a QL one), in the regions that are free by now
+    // batches' when that is a QL one), in the regions that are free by now; one that
+    // cannot be solved is reported whatever the batch, as the fused kernel does
     if (use_dc(L, n, tb, SOLVER_IMTQL2))
-      dc_chunk<T>(L, cur, nm, n, ac, wc, ic, FLAG_PH_ALL, kop, ab, q, cur, st, s);
+      dc_chunk<T>(L, cur, nm, n, ac, wc, ic, FLAG_PH_ALL, kop, 1, ab, q, cur, st, s);
     else if (n <= 8) launch_wave_only<T, 8>(cur, nm, n, ac, wc, ic, kop, st, s);
     else if (n <= 16) launch_wave_only<T, 16>(cur, nm, n, ac, wc, ic, kop, st, s);
     else if (n <= 32) launch_wave_only<T, 32>(cur, nm, n, ac, wc, ic, kop, st, s);
