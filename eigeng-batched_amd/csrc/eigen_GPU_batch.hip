@@ -1099,11 +1099,14 @@ hipError_t run(int L, int nm, int n, int m, T *a, T *w, void *wk, hipStream_t s,
   if (wk == nullptr) return hipErrorInvalidValue;
   // kernel options: solver, order of the output, eigenvector columns not stored
   const int kop = kopt_make(base, (solver & FLAG_UNSORTED) != 0, n - m);
-  if (use_dc(L, n, (int)sizeof(T), solver)) return run_dc<T>(L, nm, n, a, w, info, solver, kop, wk, s);
-  if (use_dc_large(L, n, (int)sizeof(T), solver)) return run_dc_large<T>(L, nm, n, a, w, info, solver, kop, wk, s);
-  if ((solver & FLAG_PH_ALL) && !use_split(L, n, (int)sizeof(T), solver) && !use_split_large(L, n, (int)sizeof(T), solver) &&
-      !use_split128(L, n, (int)sizeof(T), solver))
+  const int tb = (int)sizeof(T);
+  const bool dc = use_dc(L, n, tb, solver), dcl = use_dc_large(L, n, tb, solver);
+  // phases: of a batch whose QL path is one in separate kernels, or asked for with FLAG_DC
+  if ((solver & FLAG_PH_ALL) && !((dc || dcl) && (solver & FLAG_DC)) && !use_split(L, n, tb, solver) &&
+      !use_split_large(L, n, tb, solver) && !use_split128(L, n, tb, solver))
     return hipErrorInvalidValue;
+  if (dc) return run_dc<T>(L, nm, n, a, w, info, solver, kop, wk, s);
+  if (dcl) return run_dc_large<T>(L, nm, n, a, w, info, solver, kop, wk, s);
   if constexpr (sizeof(T) == 4) {
     if (use_split128(L, n, (int)sizeof(T), solver)) return launch_split<T, 128>(L, nm, n, a, w, info, solver, kop, wk, s);
   }
