@@ -233,6 +233,13 @@ bool use_dc_large(int L, int n, int tbytes, int solver)
   return (flags & FLAG_DC) || !(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L;
 }
 
+// Its chunk: FP32 n <= 128 as the QL path there, so that single phases are taken up to
+// the same batch.
+int dc_large_chunk(int n, int tbytes, int solver)
+{
+  return tbytes == 4 && n <= 128 ? lchunk(solver) : lchunk_large(solver);
+}
+
 // Its workspace for a chunk of lc matrices: the reflectors, d / e, beta, two
 // buffers of eigenvectors of T, the merges' U (later the reflector blocks' T), status.
 struct DcLargeLayout {
@@ -335,7 +342,8 @@ size_t workspace_bytes(int L, int nm, int n, int m, int tbytes, int solver)
   }
   if (use_dc_large(L, n, tbytes, solver)) {
     const size_t other = workspace_bytes(L, nm, n, m, tbytes, (solver & ~FLAG_DC) | FLAG_ROUTE_QL);
-    const size_t own = WS_HEAD + DcLargeLayout(L < lchunk_large(solver) ? L : lchunk_large(solver), n, tbytes).total;
+    const int ch = dc_large_chunk(n, tbytes, solver);
+    const size_t own = WS_HEAD + DcLargeLayout(L < ch ? L : ch, n, tbytes).total;
     return own > other ? own : other;
   }
   solver &= ~FLAG_ROUTE_QL;
@@ -1013,7 +1021,7 @@ template <typename T>
 hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver, int kop, void *wk, hipStream_t s)
 {
   constexpr int tb = (int)sizeof(T), KIND = tb == 8 ? GK_F64 : GK_F32;
-  const int lc = L < lchunk_large(solver) ? L : lchunk_large(solver);
+  const int ch = dc_large_chunk(n, tb, solver), lc = L < ch ? L : ch;
   const DcLargeLayout lay(lc, n, tb);
   char *base = (char *)wk + WS_HEAD;
   T *Wm = (T *)(base + lay.wm), *de = (T *)(base + lay.de), *bw = (T *)(base + lay.bw), *U = (T *)(base + lay.u);

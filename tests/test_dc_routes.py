@@ -2,9 +2,12 @@
 import ctypes
 
 import pytest
+import torch
 
 import eigeng_batched as eg
 
+# host memory stands for device memory: only where nothing can be launched
+pytestmark = pytest.mark.skipif(torch.cuda.device_count() > 0, reason="passes host pointers")
 PHASES = [0x1000, 0x2000, 0x4000, 0x3000]
 INVALID = 1
 
@@ -26,3 +29,15 @@ def test_phases_without_a_path_stay_refused_for_small_batches(L, n, tb, ph):
     assert refused(L, n, tb, eg.IMTQL2 | ph)
     assert refused(L, n, tb, eg.IMTQL2 | eg.FLAG_FUSED | ph)
     assert refused(L, n, tb, eg.IMTQL2 | eg.FLAG_FUSED | eg.FLAG_DC | ph)
+
+
+@pytest.mark.parametrize("L,n,tb,path", [(10000, 100, 4, 0), (16384, 65, 4, 0), (16384, 128, 4, 0),
+                                         (5000, 100, 4, 1 << eg.CHUNK_SHIFT), (16384, 48, 4, 0), (8192, 128, 8, 0)])
+def test_phases_are_taken_up_to_the_documented_batch(L, n, tb, path):
+    """FP32 n <= 128 up to 16384 matrices (a chunk bit halves that), FP64 beyond 64 up to
+    8192; one matrix more is refused."""
+    eg.tune_reset()
+    top = L if L in (16384, 8192) else (16384 if not path else 8192)
+    for ph in PHASES:
+        assert not refused(L, n, tb, eg.IMTQL2 | path | ph)
+        assert refused(top + 1, n, tb, eg.IMTQL2 | path | ph)

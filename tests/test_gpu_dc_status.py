@@ -31,3 +31,23 @@ def test_warm_start_reports_what_it_cannot_solve(n, L):
     v = z[ok].double()
     r = torch.linalg.matrix_norm(v @ a[ok].double() - w[ok].double().unsqueeze(2) * v)
     assert float((r / w[ok].double().abs().amax(1)).max()) <= 8 * n * 2.0 ** -23
+
+
+def test_large_fp32_chunk_and_its_phases():
+    """FP32 64 < n <= 128 in one chunk of more than 8192 matrices: the bits of a smaller
+    batch, and of the call phase by phase."""
+    n, L = 66, 9000
+    g = torch.Generator(device=DEV)
+    g.manual_seed(3)
+    b = torch.rand((L, n, n), generator=g, device=DEV) - 0.5
+    a = (b + b.transpose(1, 2)).contiguous()
+    z, w, info = eg.eigen_batch(a.clone())
+    z0, w0, _ = eg.eigen_batch(a[6000:].clone())
+    ws = torch.empty(eg.bufsize(L, n, n, n, 4), dtype=torch.uint8, device=DEV)
+    zp, wp = a.clone(), torch.empty_like(w)
+    for ph in ("tri", "ql", "apply"):
+        eg.eigen_batch(zp, w=wp, workspace=ws, phases=[ph])
+    torch.cuda.synchronize()
+    assert int(info.abs().max()) == 0
+    assert torch.equal(z[6000:], z0) and torch.equal(w[6000:], w0)
+    assert torch.equal(zp, z) and torch.equal(wp, w)
