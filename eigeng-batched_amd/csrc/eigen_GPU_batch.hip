@@ -1905,17 +1905,8 @@ hipError_t launch_params(int L, int n, int tb, int solver, int *p)
     p[3] = threads;
     p[1] = (nmat + g - 1) / g;
   };
-  if (use_dc(L, n, tb, solver)) {
-    grp(nb_of(n), L < lchunk(solver) ? L : lchunk(solver), 64);
-  } else if (use_dc_large(L, n, tb, solver)) {
-    const int lc = L < lchunk_large(solver) ? L : lchunk_large(solver);
-    // callers are told the shapes they always were: order class and matrices in flight
-    if (tb == 4 && n <= 128 && L >= SPLIT_MIN_L) {
-      grp(128, lc, 128);
-    } else {
-      p[0] = 256; p[1] = lc < 1024 ? lc : 1024; p[2] = 1; p[3] = 256;
-    }
-  } else if (tb == 4 && use_split128(L, n, tb, solver)) {
+  // divide and conquer is left out: the shapes of the path without it (eigen_GPU_batch.h)
+  if (tb == 4 && use_split128(L, n, tb, solver)) {
     grp(128, L < lchunk(solver) ? L : lchunk(solver), 128);
   } else if (use_split(L, n, tb, solver)) {
     grp(nb_of(n), L < lchunk(solver) ? L : lchunk(solver), 64);

@@ -500,7 +500,8 @@ def tune_set(L: int, n: int, dtype_bytes: int, bits: int, solver: int = IMTQL2) 
 
 
 def launch_params(L: int, n: int, dtype_bytes: int, solver: int = IMTQL2) -> dict:
-    """Launch shape of the first kernel a call takes (eigen_GPU_batch_launch_params)."""
+    """Order class and matrices in flight as a launch shape (eigen_GPU_batch_launch_params):
+    the first kernel of the QL or Jacobi path that fits the call."""
     p = (ctypes.c_int * 6)()
     rc = lib().eigen_GPU_batch_launch_params(L, n, dtype_bytes, solver, ctypes.addressof(p))
     keys = ("grpSZ", "numTB", "numGR", "numTH", "sizeSH", "sizeL2")

@@ -273,14 +273,17 @@ int eigen_GPU_batch_gram_DP(int L, int nm, int n, int p, const double *y, int ld
                             hipStream_t stream);
 
 /*
- * Launch shape of the first kernel of the path a call with (L, n, element
- * size, solver) takes (tuning included), in the terms of the reference's
- * eigen_GPU_batch_get_Launch_params (eigen_GPU_batch.hpp:23-102): params[0]
- * lanes per matrix group, [1] workgroups, [2] matrices (groups) per
- * workgroup, [3] threads per workgroup, [4] dynamic LDS bytes passed at
- * launch (0: the kernels size their LDS statically), [5] L2 bytes of the
- * current device.  Returns hipSuccess, or hipErrorInvalidValue /
- * hipErrorNotSupported with params zeroed.
+ * Launch shape of a call with (L, n, element size, solver), tuning included, in
+ * the terms of the reference's eigen_GPU_batch_get_Launch_params
+ * (eigen_GPU_batch.hpp:23-102), as that of the first kernel of the QL or Jacobi
+ * path that fits the call: params[0] lanes per matrix group, [1] workgroups,
+ * [2] matrices (groups) per workgroup, [3] threads per workgroup, [4] dynamic
+ * LDS bytes passed at launch (0: the kernels size their LDS statically), [5] L2
+ * bytes of the current device.  They are the order class and the matrices in
+ * flight for callers that size by them, not a record of the launch: where the
+ * call takes divide and conquer, or the register-resident tridiagonalisation for
+ * 64 < n <= 256, the grid and the workgroup are others.  Returns hipSuccess, or
+ * hipErrorInvalidValue / hipErrorNotSupported with params zeroed.
  */
 int eigen_GPU_batch_launch_params(int L, int n, int dtype_bytes, int solver, int *params);
 

@@ -41,3 +41,15 @@ def test_phases_are_taken_up_to_the_documented_batch(L, n, tb, path):
     for ph in PHASES:
         assert not refused(L, n, tb, eg.IMTQL2 | path | ph)
         assert refused(top + 1, n, tb, eg.IMTQL2 | path | ph)
+
+
+@pytest.mark.parametrize("tb", [4, 8])
+def test_launch_params_are_those_of_the_path_without_divide_and_conquer(tb):
+    """The same numbers with and without it (bit 28 means nothing to IMTQL2 but keeps a
+    call off that path)."""
+    eg.tune_reset()
+    for L in (1, 100, 257, 600, 1024, 2048, 8192, 16384):
+        for n in (5, 8, 20, 32, 48, 64, 65, 100, 128, 129, 192, 200, 256, 257, 300, 512):
+            p = eg.launch_params(L, n, tb)
+            assert p["rc"] == 0
+            assert p == eg.launch_params(L, n, tb, eg.IMTQL2 | (1 << 28)) == eg.launch_params(L, n, tb, eg.FLAG_DC)
