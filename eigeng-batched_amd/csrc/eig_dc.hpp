@@ -28,9 +28,10 @@
 //      working precision without extended arithmetic.
 //   4. the new eigenvalues are ranked, the vectors U formed in that order, and
 //      Q <- Q U on the matrix cores.
-// Steps 1-3 run on the node scaled by a power of two to a largest entry of order one,
-// whatever its size against the rest of T: the products of step 3 hold one factor of
-// (node's size) / HUGE_, and the derivative in step 2 is of the order of 1 / size.
+// Steps 1-3 run on nodes of order one: one that is smaller than the rest of T by more
+// than DcLim::NODE is scaled by a power of two, since the products of step 3 hold one
+// factor of (node's size) / HUGE_ and the derivative in step 2 is of the order of
+// 1 / size (FP32: vectors off by order one from a size of 1e-16 on).
 #pragma once
 #include "common.hpp"
 #include "eig_symdmt.hpp"
@@ -38,16 +39,16 @@
 
 namespace eigmi {
 
-// HUGE_ (a node is scaled to a largest entry of order one): from here on a value
+// HUGE_ (a node's largest entry is between NODE and order one): from here on a value
 // stands for "no pole"; slot p of a node uses HUGE_ (1 + p / 1024), so that
 // these sort behind the poles in the order of their slots.  STEP: 4 sqrt(eps).
 template <typename T> struct DcLim;
 template <> struct DcLim<float> {
-  static constexpr float HUGE_ = 1e18f, STEP = 1.3810679e-03f;
+  static constexpr float HUGE_ = 1e18f, STEP = 1.3810679e-03f, NODE = 1e-6f;
   static constexpr int EXP = 120;                       // scale factors stay normal
 };
 template <> struct DcLim<double> {
-  static constexpr double HUGE_ = 1e150, STEP = 5.9604644775390625e-08;
+  static constexpr double HUGE_ = 1e150, STEP = 5.9604644775390625e-08, NODE = 1e-6;
   static constexpr int EXP = 1000;
 };
 
@@ -347,6 +348,7 @@ struct alignas(16) DcLds {
   alignas(16) T ma[NB], mt[NB];                  // root by new column
   alignas(16) int src[NB], mdef[NB];             // column that passes through, by slot / new column (-1: a root)
   alignas(16) T e[NB];
+  alignas(16) int ex[NB];                        // exponent of the scale of a column's node
   alignas(16) T red[4];
   int flag[4];
 };
@@ -462,12 +464,12 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
   const int end = (base + S < n) ? base + S : n;               // live columns of the node end here
   const bool both = mid < n;                                   // the node has a right child
   // ---- 1. z, the poles set aside, ranks --------------------------------------
-  T z = T(0), rho = T(0), key = HUGE_, dmax = T(0), sc = T(1);
-  bool nd = false;
-  int c = 0, k = 0, ex = 0;
+  T z = T(0), rho = T(0), key = HUGE_, dmax = T(0);
+  bool nd = false, small = false;                              // small: a node of this wave is scaled
+  int c = 0, k = 0;
   if (on) {
     const T er = both ? Sh.e[mid - 1] : T(0);
-    const T di = Sh.d[i];
+    T di = Sh.d[i];
     rho = abs_(er);
     z = (i < mid) ? Sh.B[fb][i] : sign_(T(1), er) * Sh.F[fb][i];
     dmax = rho;
@@ -476,14 +478,20 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
       dmax = max_(dmax, max_(abs_(Sh.d[base]), abs_(Sh.d[(both ? mid : end) - 1])));
       if (both) dmax = max_(dmax, max_(abs_(Sh.d[mid]), abs_(Sh.d[end - 1])));
     }
-    // steps 1-3 on the node scaled to order one (a power of two: exact)
-    if (dmax > T(0)) (void)frexp(dmax, &ex);
-    ex = max(min(ex, DcLim<T>::EXP), -DcLim<T>::EXP);
-    sc = ldexp(T(1), -ex);
-    rho *= sc;
-    dmax *= sc;
+    // steps 1-3 on a small node scaled to order one (a power of two: exact)
+    const bool tiny = dmax > T(0) && dmax < DcLim<T>::NODE;
+    small = __ballot(tiny) != 0ull;
+    if (small) {
+      int ex = 0;
+      if (tiny) (void)frexp(dmax, &ex);
+      ex = max(ex, -DcLim<T>::EXP);
+      rho = ldexp(rho, -ex);
+      dmax = ldexp(dmax, -ex);
+      di = ldexp(di, -ex);
+      Sh.ex[i] = ex;
+    }
     nd = i < n && rho * abs_(z) > T(2) * eps * dmax;
-    key = nd ? di * sc : HUGE_ * (T(1) + T(p) * T(1.0 / 1024));
+    key = nd ? di : HUGE_ * (T(1) + T(p) * T(1.0 / 1024));
     if (sub == 0) Sh.key[i] = key;
   }
   dc_sync<LW>();
@@ -556,11 +564,9 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
     dc_root<T, S, LN, REG>(&Sh.dl[base], &Sh.zq[base], k, p, sub, rho, root, a0, t0);
     if (root) { da = a0; tau = t0; }
     s0 = Sh.src[i] & 63;
-    if (s0 >= n) {                                             // no column: HUGE_ in every scale
-      sc = T(1);
-      ex = 0;
-    }
-    v0 = root ? da + tau : Sh.d[s0] * sc;
+    v0 = root ? da + tau : Sh.d[s0];
+    // (a slot without a column keeps HUGE_ in every scale)
+    if (small && !root && s0 < n) v0 = ldexp(v0, -Sh.ex[i]);
     if (sub == 0) {
       Sh.da[i] = da;
       Sh.tau[i] = tau;
@@ -594,7 +600,8 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
       Sh.ma[nr] = da;
       Sh.mt[nr] = tau;
       Sh.mdef[nr] = root ? -1 : s0;
-      Sh.d[nr] = ldexp(v0, ex);   // every read of the old values is before the last barrier
+      // every read of the old values is before the last barrier
+      Sh.d[nr] = (small && s0 < n) ? ldexp(v0, Sh.ex[i]) : v0;
     }
   }
   dc_sync<NW>();
