@@ -120,10 +120,12 @@ template <int S, int NLR> struct DcDeal {
 // distinct, zq = z^2 > 0, entries k.. of d HUGE_ and of zq zero: lambda = da + tau.
 // All lanes of the wave call it (`live`: this one has a root).  REG: the lane's
 // poles and weights stay in registers, otherwise every evaluation reads them
-// from LDS.
+// from LDS.  False where maxit evaluations (DC_MAXIT; the most seen is 21) did not end
+// in a root.
+constexpr int DC_MAXIT = 64;
 template <typename T, int S, int NLR, bool REG>
-__device__ __forceinline__ void dc_root(const T *__restrict__ dl, const T *__restrict__ zq, int k, int p, int sub,
-                                        T rho, bool live, T &da_out, T &tau_out)
+__device__ __forceinline__ bool dc_root(const T *__restrict__ dl, const T *__restrict__ zq, int k, int p, int sub,
+                                        T rho, bool live, int maxit, T &da_out, T &tau_out)
 {
   constexpr int NQ = DcDeal<S, NLR>::NQ;
   const T eps = eps_of<T>();
@@ -217,7 +219,7 @@ __device__ __forceinline__ void dc_root(const T *__restrict__ dl, const T *__res
   const T o1 = last ? gl : (left ? T(0) : -gap), o2 = last ? T(0) : (left ? gap : T(0));
   bool act = live;
 #pragma unroll 1
-  for (int it = 0; it < 64; ++it) {
+  for (int it = 0; it < maxit; ++it) {
     if (!__ballot(act)) break;
     // w: the sum; as: of absolute values; dal: its derivative; sd: the
     // derivative's terms right of the root minus those left of it
@@ -290,6 +292,7 @@ __device__ __forceinline__ void dc_root(const T *__restrict__ dl, const T *__res
   }
   da_out = da;
   tau_out = tau;
+  return !act;
 }
 
 // z of pole p recomputed from the roots, squared, up to a factor that is the
@@ -351,6 +354,7 @@ struct alignas(16) DcLds {
   alignas(16) int ex[NB];                        // exponent of the scale of a column's node
   alignas(16) T red[4];
   int flag[4];
+  int lost;                                      // a root was not found or a vector came to nothing
 };
 
 template <int NW>
@@ -443,10 +447,11 @@ __device__ __forceinline__ void dc_apply(const T *__restrict__ aop, int lane, ty
 // the workgroup's lanes per column; with fewer, the first waves do steps 1-3
 // alone): an evaluation costs about 7 instructions a pole and 45 more, so small
 // nodes take one lane a root and large ones the whole workgroup.
+// Returns DcLds::lost of all levels so far.
 template <typename T, int NB, int NLR, int S, int H, int LN>
-__device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
+__device__ __forceinline__ bool dc_merge_level(DcLds<NB, T> &Sh,
                                                typename Mfma16<T>::v4 (&X)[DcShape<NB, NLR>::CT][NB / 16], int n,
-                                               int fb)
+                                               int fb, int maxit)
 {
   typedef DcShape<NB, NLR> G;
   typedef DcDeal<S, LN> Deal;
@@ -557,11 +562,12 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
   }
   // ---- 2. roots ----------------------------------------------------------------
   const bool root = on && p < k;
+  bool ok = true;
   T da = HUGE_, tau = T(0), v0 = T(0);
   int s0 = 0;
   if (on) {
     T a0, t0;
-    dc_root<T, S, LN, REG>(&Sh.dl[base], &Sh.zq[base], k, p, sub, rho, root, a0, t0);
+    ok = dc_root<T, S, LN, REG>(&Sh.dl[base], &Sh.zq[base], k, p, sub, rho, root, maxit, a0, t0);
     if (root) { da = a0; tau = t0; }
     s0 = Sh.src[i] & 63;
     v0 = root ? da + tau : Sh.d[s0];
@@ -577,6 +583,7 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
   // ---- 3. z from the roots; new order -------------------------------------------
   if (on) {
     const T z2 = dc_zhat2<T, S, LN, REG>(&Sh.dl[base], &Sh.da[base], &Sh.tau[base], k, root ? p : 0, sub);
+    if (root && !(ok && z2 > T(0) && finite_(z2))) Sh.lost = 1;     // (an offset of zero gives a z of zero)
     // without a column set aside the roots are in order already
     int nr = p;
     if (__ballot(base + k < end)) {
@@ -605,6 +612,7 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
     }
   }
   dc_sync<NW>();
+  const int lost = __builtin_amdgcn_readfirstlane(Sh.lost);
   // ---- 4. U (A operand: lane = new column, slots = old columns) -------------------
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
@@ -652,6 +660,7 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
   // ---- 5. X <- U^T X ----------------------------------------------------------------
   dc_apply<T, NB, CT, TS>(Sh.aop, lane, X);
   if (!LAST) dc_sync<NW>();
+  return lost != 0;
 }
 
 // Full solve after the tridiagonalisation for n <= NB (NB = 16, 32, 48, 64): Q
@@ -660,7 +669,9 @@ __device__ __forceinline__ void dc_merge_level(DcLds<NB, T> &Sh,
 // eigenvectors of A themselves.
 // BLK: a 64-column block of a larger matrix (nblk per matrix) with X starting from
 // the identity: the block's eigenvectors of T to z0 or z1 (bit b of zmask; ld n,
-// at (64 b, 64 b)) and its eigenvalues to w (NaN for a block that is not finite).
+// at (64 b, 64 b)) and its eigenvalues to w (NaN for a block that is not finite,
+// infinities for one whose merges failed).
+// A matrix whose merges failed (DcLds::lost): info = 1 and a untouched.
 // nanfail: what a matrix that is not finite gives: 1: info = 1 and a untouched,
 // 0: the diagonal and Q as they are (sorted by the reference's rule), info = 0
 // (the two outcomes of the QL paths, by batch size).
@@ -775,6 +786,7 @@ __global__ __launch_bounds__(NB *NLR) __attribute__((amdgpu_waves_per_eu(DcTune<
       Sh.key[i] = lv ? dv * sc : T(0);
       Sh.e[i] = ev * sc;
     }
+    if (tid == 0) Sh.lost = 0;
     if (tid < 64) {
       // entries beyond the block never hold a pole
       if (tid >= NB) {
@@ -827,16 +839,18 @@ __global__ __launch_bounds__(NB *NLR) __attribute__((amdgpu_waves_per_eu(DcTune<
     dc_apply<T, NB, CT, 1>(Sh.aop, lane, X);
     dc_sync<NW>();
   }
+  const int maxit = kopt_cut(opts) ? 1 : DC_MAXIT;
   constexpr int L1 = NB >= 48 ? 1 : (NB == 32 ? 2 : NLR), L2 = NB >= 48 ? 2 : NLR;
-  dc_merge_level<T, NB, NLR, 4, 2, L1>(Sh, X, n, 0);
-  dc_merge_level<T, NB, NLR, 8, 4, L1>(Sh, X, n, 1);
-  dc_merge_level<T, NB, NLR, 16, 8, L1>(Sh, X, n, 0);
-  if constexpr (NB >= 32) dc_merge_level<T, NB, NLR, 32, 16, L2>(Sh, X, n, 1);
-  if constexpr (NB == 48) dc_merge_level<T, NB, NLR, 48, 32, NLR>(Sh, X, n, 0);
-  if constexpr (NB == 64) dc_merge_level<T, NB, NLR, 64, 32, NLR>(Sh, X, n, 0);
+  dc_merge_level<T, NB, NLR, 4, 2, L1>(Sh, X, n, 0, maxit);
+  dc_merge_level<T, NB, NLR, 8, 4, L1>(Sh, X, n, 1, maxit);
+  bool lost = dc_merge_level<T, NB, NLR, 16, 8, L1>(Sh, X, n, 0, maxit);
+  if constexpr (NB >= 32) lost = dc_merge_level<T, NB, NLR, 32, 16, L2>(Sh, X, n, 1, maxit);
+  if constexpr (NB == 48) lost = dc_merge_level<T, NB, NLR, 48, 32, NLR>(Sh, X, n, 0, maxit);
+  if constexpr (NB == 64) lost = dc_merge_level<T, NB, NLR, 64, 32, NLR>(Sh, X, n, 0, maxit);
 
-  if (sub == 0 && lv) wout[i] = Sh.d[i] * isc;
-  if (!BLK && info && tid == 0) info[mat] = 0;
+  if (sub == 0 && lv) wout[i] = (BLK && lost) ? std::numeric_limits<T>::infinity() : Sh.d[i] * isc;
+  if (!BLK && info && tid == 0) info[mat] = lost ? 1 : 0;
+  if (!BLK && lost) return;
   T *__restrict__ O = BLK ? (((zmask >> (b0 / 64)) & 1) ? z1 : z0) + (size_t)mat * n_all * n_all + (size_t)b0 * n_all + b0
                           : a + (size_t)mat * (size_t)nm * (size_t)n;
   const int ldo = BLK ? n_all : nm, mcols = BLK ? n : n - kopt_mdrop(opts);

@@ -31,17 +31,19 @@ struct alignas(16) DcMergeLds {
   alignas(16) T zk[S], dk[S], ma[S], mt[S];
   alignas(16) int src[S], mdef[S];
   int flag[16];
+  int lost;                                        // as in DcLds
 };
 
 // One workgroup per (matrix, node).  w: the eigenvalues of the blocks, replaced by
 // the nodes'.  Zc: the children's vectors.  U: the node's vectors, at (base, base)
-// of an n x n slot.  The last level (st not null) reports per matrix: st = 1
-// leaves the matrix out of the final products (not finite and nanfail), info.
+// of an n x n slot.  A node that fails leaves infinities for its eigenvalues.  The last
+// level (st not null) reports per matrix: st = 1 leaves the matrix out of the final
+// products (a merge failed, or not finite and nanfail), info.
 template <typename T, int S, int NLR>
 __global__ __launch_bounds__(S *NLR) void eig_dc_merge_kernel(int n, DcNodes nodes, const T *__restrict__ de, int ld,
                                                               T *__restrict__ w, const T *__restrict__ Zc,
                                                               T *__restrict__ U, int *__restrict__ st,
-                                                              int *__restrict__ info, int nanfail)
+                                                              int *__restrict__ info, int nanfail, int maxit)
 {
   constexpr int NTH = S * NLR, NW = NTH / 64;
   __shared__ DcMergeLds<T, S> Sh;
@@ -61,22 +63,24 @@ __global__ __launch_bounds__(S *NLR) void eig_dc_merge_kernel(int n, DcNodes nod
   if (lv) z = (i < h) ? Z[(size_t)(base + i) * n + base + h - 1] : Z[(size_t)(base + i) * n + base + h];
   // the children are sorted, so their ends bound them
   const T q0 = abs_(wm[0]), q1 = abs_(wm[h - 1]), q2 = abs_(wm[h]), q3 = abs_(wm[s - 1]);
-  bool bad = !finite_(d0) || !finite_(z) || !finite_(er0);
-  if (__ballot(bad)) bad = true;
-  if (lane == 0) Sh.flag[wv] = bad ? 1 : 0;
+  const bool bad = !finite_(d0) || !finite_(z) || !finite_(er0);
+  const int code = (__ballot(bad) != 0ull ? 1 : 0) | (__ballot(abs_(d0) == std::numeric_limits<T>::infinity()) != 0ull ? 2 : 0);
+  if (lane == 0) Sh.flag[wv] = code;
+  if (tid == 0) Sh.lost = 0;
   __syncthreads();
-  bad = false;
+  int codes = 0;
 #pragma unroll
-  for (int q = 0; q < NW; ++q) bad = bad || Sh.flag[q] != 0;
-  if (bad) {
-    // everything of this node: NaN (the products spread it)
+  for (int q = 0; q < NW; ++q) codes |= Sh.flag[q];
+  if (codes) {
+    // everything of this node: NaN (the products spread it), or infinite where a merge failed
     const T nan = std::numeric_limits<T>::quiet_NaN();
-    if (lv && sub == 0) wm[i] = nan;
+    const bool fail = nanfail || (codes & 2);
+    if (lv && sub == 0) wm[i] = (codes & 2) ? std::numeric_limits<T>::infinity() : nan;
     for (int m = wv; m < s; m += NW)
       for (int k = lane; k < s; k += 64) Um[(size_t)m * n + k] = nan;
     if (st && tid == 0) {
-      st[mat] = nanfail ? 1 : 0;
-      if (info) info[mat] = nanfail ? 1 : 0;
+      st[mat] = fail ? 1 : 0;
+      if (info) info[mat] = fail ? 1 : 0;
     }
     return;
   }
@@ -156,10 +160,11 @@ __global__ __launch_bounds__(S *NLR) void eig_dc_merge_kernel(int n, DcNodes nod
   }
   // ---- 2. roots --------------------------------------------------------------------
   const bool root = i < k;
+  bool ok = true;
   T da = HUGE_, tau = T(0);
   {
     T a0 = T(0), t0 = T(0);
-    if (__ballot(root)) dc_root<T, S, NLR, false>(Sh.dl, Sh.zq, k, i, sub, rho, root, a0, t0);
+    if (__ballot(root)) ok = dc_root<T, S, NLR, false>(Sh.dl, Sh.zq, k, i, sub, rho, root, maxit, a0, t0);
     if (root) { da = a0; tau = t0; }
   }
   const int s0 = Sh.src[i] & (S - 1);
@@ -174,6 +179,7 @@ __global__ __launch_bounds__(S *NLR) void eig_dc_merge_kernel(int n, DcNodes nod
   {
     T z2 = T(0);
     if (__ballot(root)) z2 = dc_zhat2<T, S, NLR, false>(Sh.dl, Sh.da, Sh.tau, k, root ? i : 0, sub);
+    if (root && !(ok && z2 > T(0) && finite_(z2))) Sh.lost = 1;
     int nr = i;
     if (k < s) {
       nr = 0;
@@ -197,11 +203,13 @@ __global__ __launch_bounds__(S *NLR) void eig_dc_merge_kernel(int n, DcNodes nod
       if (nr < s) wm[nr] = v0 * isc;
     }
   }
-  if (st && tid == 0) {
-    st[mat] = 0;
-    if (info) info[mat] = 0;
-  }
   __syncthreads();
+  const bool lost = Sh.lost != 0;
+  if (st && tid == 0) {
+    st[mat] = lost ? 1 : 0;
+    if (info) info[mat] = lost ? 1 : 0;
+  }
+  if (lost && lv && sub == 0) wm[i] = std::numeric_limits<T>::infinity();
   // ---- 4. U, one column per wave at a time ----------------------------------------------
   for (int m = wv; m < s; m += NW) {
     const T a = Sh.ma[m], t0 = Sh.mt[m];

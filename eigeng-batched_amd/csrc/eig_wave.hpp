@@ -36,7 +36,8 @@ constexpr int ST_OVERFLOW = -2;
 // Output options packed with the solver id into the kernels' `solver`
 // argument: bits 0-7 the solver, bit 8 keep the QL / Jacobi order of the
 // eigenpairs (the reference's DO_SORT 0, eigen_GPU_batch.cu:5,10), bits 12-21
-// the number of trailing eigenvector columns not written (n - m).  Launches
+// the number of trailing eigenvector columns not written (n - m); bit 9 (divide
+// and conquer) one evaluation a root, so that the merges fail.  Launches
 // that pass a bare solver id get the default: sorted, all n columns.
 __host__ __device__ constexpr int kopt_make(int solver, bool unsorted, int mdrop)
 {
@@ -44,6 +45,8 @@ __host__ __device__ constexpr int kopt_make(int solver, bool unsorted, int mdrop
 }
 __host__ __device__ constexpr int kopt_solver(int o) { return o & 0xff; }
 __host__ __device__ constexpr bool kopt_unsorted(int o) { return ((o >> 8) & 1) != 0; }
+constexpr int KOPT_CUT = 0x200;
+__host__ __device__ constexpr bool kopt_cut(int o) { return (o & KOPT_CUT) != 0; }
 __host__ __device__ constexpr int kopt_mdrop(int o) { return (o >> 12) & 0x3ff; }   // split path: rotation log full, solve with the fused kernel
 
 // Offset of packed Householder column c (1 <= c) when column c' holds

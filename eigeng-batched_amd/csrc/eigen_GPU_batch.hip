@@ -214,12 +214,18 @@ int dc_max_l(int n, int tbytes)
 }
 // FLAG_SPLIT asks for the path in separate kernels: on batches that take it by
 // themselves that is this one, smaller ones get the QL recurrence.
+// FLAG_DC with FLAG_TINYLOG: the merges cut short so that they fail (a host-forced test).
+bool dc_bits(int solver)
+{
+  int flags = solver & ~0xff & ~(3 << CHUNK_SHIFT) & ~FLAG_PH_ALL;
+  if ((flags & (FLAG_DC | FLAG_SPLIT)) == FLAG_DC) flags &= ~FLAG_TINYLOG;
+  return (solver & 0xff) == SOLVER_IMTQL2 && !(flags & ~(FLAG_DC | FLAG_SPLIT));
+}
 bool use_dc(int L, int n, int tbytes, int solver)
 {
-  const int flags = solver & ~0xff & ~(3 << CHUNK_SHIFT) & ~FLAG_PH_ALL;
-  if ((solver & 0xff) != SOLVER_IMTQL2 || (flags & ~(FLAG_DC | FLAG_SPLIT)) || n > 64) return false;
-  if (flags & FLAG_DC) return true;
-  return n >= DC_MIN_N && L <= dc_max_l(n, tbytes) && (!(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L);
+  if (!dc_bits(solver) || n > 64) return false;
+  if (solver & FLAG_DC) return true;
+  return n >= DC_MIN_N && L <= dc_max_l(n, tbytes) && (!(solver & FLAG_SPLIT) || L >= SPLIT_MIN_L);
 }
 
 // 64 < n <= 512, the same interface: reflectors and a blocked back-transformation.
@@ -228,9 +234,8 @@ bool use_dc(int L, int n, int tbytes, int solver)
 bool use_dc_large(int L, int n, int tbytes, int solver)
 {
   (void)tbytes;
-  const int flags = solver & ~0xff & ~(3 << CHUNK_SHIFT) & ~FLAG_PH_ALL;
-  if ((solver & 0xff) != SOLVER_IMTQL2 || (flags & ~(FLAG_DC | FLAG_SPLIT)) || n <= 64 || n > GL_NMAX) return false;
-  return (flags & FLAG_DC) || !(flags & FLAG_SPLIT) || L >= SPLIT_MIN_L;
+  if (!dc_bits(solver) || n <= 64 || n > GL_NMAX) return false;
+  return (solver & FLAG_DC) || !(solver & FLAG_SPLIT) || L >= SPLIT_MIN_L;
 }
 
 // Its chunk: FP32 n <= 128 as the QL path there, so that single phases are taken up to
@@ -1030,6 +1035,7 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
   const int ph = (solver & FLAG_PH_ALL) ? (solver & FLAG_PH_ALL) : FLAG_PH_ALL;
   if (ph != FLAG_PH_ALL && L > lc) return hipErrorInvalidValue;
   const int nanfail = L < (tb == 4 && n <= 128 ? SPLIT_MIN_L : SPLIT_LARGE_MIN_L) ? 1 : 0;
+  const int maxit = kopt_cut(kop) ? 1 : DC_MAXIT;
   const int nblk = (n + 63) / 64, nb16 = (n + 15) / 16, mcols = n - kopt_mdrop(kop);
   DcNodes lev[4] = {};
   int levels = 0, zmask = 0;
@@ -1067,13 +1073,13 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
         int *sd = d == 0 ? st : nullptr;
         if (big <= 128)
           hipLaunchKernelGGL((eig_dc_merge_kernel<T, 128, 4>), dim3(grid), dim3(512), 0, s, n, l, (const T *)de, lc, wc,
-                             Zc, U, sd, ic, nanfail);
+                             Zc, U, sd, ic, nanfail, maxit);
         else if (big <= 256)
           hipLaunchKernelGGL((eig_dc_merge_kernel<T, 256, 4>), dim3(grid), dim3(1024), 0, s, n, l, (const T *)de, lc,
-                             wc, Zc, U, sd, ic, nanfail);
+                             wc, Zc, U, sd, ic, nanfail, maxit);
         else
           hipLaunchKernelGGL((eig_dc_merge_kernel<T, 512, 2>), dim3(grid), dim3(1024), 0, s, n, l, (const T *)de, lc,
-                             wc, Zc, U, sd, ic, nanfail);
+                             wc, Zc, U, sd, ic, nanfail, maxit);
         hipLaunchKernelGGL((eig_dc_update_kernel<T>), dim3((unsigned)cur * (unsigned)tiles), dim3(GM_THREADS), 0, s,
                            cur, n, l, tiles, Zc, (const T *)U, Z[d & 1]);
       }
@@ -1106,13 +1112,14 @@ hipError_t run(int L, int nm, int n, int m, T *a, T *w, void *wk, hipStream_t s,
   if (base != SOLVER_IMTQL2 && base != SOLVER_TQL2 && base != SOLVER_JACOBI) return hipErrorNotSupported;
   if (wk == nullptr) return hipErrorInvalidValue;
   // kernel options: solver, order of the output, eigenvector columns not stored
-  const int kop = kopt_make(base, (solver & FLAG_UNSORTED) != 0, n - m);
+  int kop = kopt_make(base, (solver & FLAG_UNSORTED) != 0, n - m);
   const int tb = (int)sizeof(T);
   const bool dc = use_dc(L, n, tb, solver), dcl = use_dc_large(L, n, tb, solver);
   // phases: of a batch whose QL path is one in separate kernels, or asked for with FLAG_DC
   if ((solver & FLAG_PH_ALL) && !((dc || dcl) && (solver & FLAG_DC)) && !use_split(L, n, tb, solver) &&
       !use_split_large(L, n, tb, solver) && !use_split128(L, n, tb, solver))
     return hipErrorInvalidValue;
+  if ((dc || dcl) && (solver & FLAG_TINYLOG)) kop |= KOPT_CUT;
   if (dc) return run_dc<T>(L, nm, n, a, w, info, solver, kop, wk, s);
   if (dcl) return run_dc_large<T>(L, nm, n, a, w, info, solver, kop, wk, s);
   if constexpr (sizeof(T) == 4) {

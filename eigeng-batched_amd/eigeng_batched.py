@@ -182,7 +182,8 @@ def eigen_batch(a, w=None, m: int | None = None, solver: int = IMTQL2, info=None
 
     Returns (a, w, info): eigenvectors overwrite ``a`` (column j of matrix k is
     ``a[k, j, :n]``), ``w`` (L, n) ascending eigenvalues, ``info`` (L,) int32
-    per-matrix status (0 ok, l>0 QL did not converge) or None when abi=True.
+    per-matrix status (0 ok, l>0 QL did not converge or, 1, a merge of divide and
+    conquer failed) or None when abi=True.
     abi=True calls the reference-compatible eigen_GPU_batch_FP/_DP symbol.
     path selects the n <= 64 implementation: "auto", "fused" (one kernel), "dc"
     (divide and conquer, what "auto" takes for most shapes), "split" (separate

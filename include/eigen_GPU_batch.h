@@ -97,6 +97,8 @@ enum eigen_GPU_batch_solver {
  *   0x8000000 (IMTQL2) divide and conquer whatever the shape, n <= 512;
  *   0x400  (with 0x200) shrink the rotation log so every matrix takes the
  *          split path's overflow fallback (a host-forced test of that path);
+ *          (with 0x8000000 alone) cut the merges of divide and conquer short so
+ *          that they fail (a host-forced test of its status);
  *   0x1000 / 0x2000 / 0x4000  run only the tridiagonalisation / QL (or merges) /
  *          apply phase of a path in separate kernels (L <= 16384): successive calls on one stream with
  *          one workspace compose the full solve, so each phase can be timed;
@@ -136,7 +138,12 @@ size_t eigen_GPU_batch_bufsize(int L, int nm, int n, int m, int dtype_bytes, int
  * optional per-matrix status array `info` (device int[L], may be NULL):
  * info[k] = 0 on success, l >= 1 if the QL iteration for eigenvalue l did not
  * converge in 100 sweeps (eigenvalues then unsorted, eigenvectors not written),
- * as the reference's ierror (tql2_tiled.hpp:138).  Returns hipSuccess, or
+ * as the reference's ierror (tql2_tiled.hpp:138); with divide and conquer 1 if a
+ * merge failed (a root not found in 64 evaluations, or a vector without a finite
+ * norm; eigenvalues then undefined, eigenvectors not written).  A matrix that is
+ * not finite, or whose reduction over- or underflows, is reported by the paths of
+ * small batches (info 1, eigenvectors not written); those of large ones return
+ * NaN with info 0.  Returns hipSuccess, or
  * hipErrorInvalidValue for invalid arguments (nothing launched), or the launch
  * error.  wk must hold eigen_GPU_batch_bufsize(...) bytes.
  */

@@ -51,3 +51,23 @@ def test_large_fp32_chunk_and_its_phases():
     assert int(info.abs().max()) == 0
     assert torch.equal(z[6000:], z0) and torch.equal(w[6000:], w0)
     assert torch.equal(zp, z) and torch.equal(wp, w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,L", [(8, 40), (16, 3000), (20, 40), (20, 600), (40, 40), (64, 2100), (65, 40), (100, 2100),
+                                 (200, 40), (300, 8), (512, 4)])
+def test_merges_that_fail_are_reported(n, L, dtype):
+    """One evaluation a root (0x8000000 with 0x400): a matrix with roots to find is
+    reported in info and left as it was, a diagonal one is solved."""
+    print(f"[dc lost] n={n} L={L} {dtype}", flush=True)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(n)
+    b = torch.rand((L, n, n), generator=g, device=DEV, dtype=dtype) - 0.5
+    a = (b + b.transpose(1, 2)).contiguous()
+    a[1::2] = torch.diag_embed(torch.diagonal(a[1::2], dim1=1, dim2=2))
+    z, w, info = eg.eigen_batch(a.clone(), solver=eg.IMTQL2 | 0x400, path="dc")
+    torch.cuda.synchronize()
+    assert bool((info[0::2] == 1).all()) and torch.equal(z[0::2], a[0::2])
+    assert int(info[1::2].abs().max()) == 0
+    assert torch.equal(w[1::2], torch.diagonal(a[1::2], dim1=1, dim2=2).sort(dim=1)[0])
+    assert torch.equal(z[1::2].abs().sum(2), torch.ones_like(w[1::2]))
