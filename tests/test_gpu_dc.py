@@ -115,6 +115,8 @@ def test_more_matrices_than_workgroups(n, dtype):
     assert torch.equal(w.view(206, *w0.shape), w0.expand(206, *w0.shape))
 
 
+# Q is formed explicitly nowhere for n > 64 any more: these batches take the reflectors and
+# the blocked back-transformation as smaller ones do, and no small batch is compared with.
 @pytest.mark.parametrize("n", [65, 100, 128])
 def test_families_with_explicit_q(n):
     """FP32 batches of 2048 and more, n <= 128: Q formed by the tridiagonalisation
@@ -150,6 +152,8 @@ def test_first_columns_and_smaller_chunks(n, dtype):
     assert torch.equal(w, wp) and torch.equal(z, zp)
 
 
+# From 2048 matrices on, "split" is divide and conquer itself for n <= 64:
+# test_gpu_dc_status.py compares with routes that are QL at every size.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("n,L", [(20, 40), (20, 3000), (48, 100), (48, 2100), (64, 30), (100, 60), (100, 2050),
                                  (200, 30), (200, 520)])

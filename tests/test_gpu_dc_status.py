@@ -71,3 +71,69 @@ def test_merges_that_fail_are_reported(n, L, dtype):
     assert int(info[1::2].abs().max()) == 0
     assert torch.equal(w[1::2], torch.diagonal(a[1::2], dim1=1, dim2=2).sort(dim=1)[0])
     assert torch.equal(z[1::2].abs().sum(2), torch.ones_like(w[1::2]))
+
+
+def ql_route(n, L, dtype):
+    """A route of the QL recurrence with the outcome of the path a batch took without
+    divide and conquer (extra bits keep it off that path): (path, extra solver bits)."""
+    f32 = dtype == torch.float32
+    if n <= 64:
+        least = 1 if 16 <= n <= 32 and not f32 or 28 <= n <= 32 else 1024 if f32 and n >= 56 else 2048
+        return ("split-lds", 0) if L >= least else ("fused", 0)
+    if f32 and n <= 128:
+        return ("split-reg128", 0) if L >= 2048 else ("fused", 0)
+    if L < 512:
+        return ("fused", 0)
+    return ("split-ws", 0) if n <= 256 else ("split", 1 << 28)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,L", [(8, 40), (8, 3000), (12, 3000), (20, 40), (20, 3000), (30, 40), (48, 100), (48, 2100),
+                                 (60, 1500), (64, 30), (64, 2100), (100, 60), (100, 2050), (200, 30), (200, 520),
+                                 (300, 30)])
+def test_statuses_of_matrices_that_are_not_finite(n, L, dtype):
+    """A NaN or an infinity: the status of the QL route, NaN among the eigenvalues of both,
+    and for n <= 64 the same eigenvectors written or left."""
+    path, extra = ql_route(n, L, dtype)
+    print(f"[dc status] n={n} L={L} {dtype} against {path}", flush=True)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(7)
+    b = torch.rand((L, n, n), generator=g, device=DEV, dtype=dtype) - 0.5
+    a = (b + b.transpose(1, 2)).contiguous()
+    bad = [1, 7, 20, 25]
+    a[1] = float("nan")
+    a[7, 5, 3] = float("nan")
+    a[20, 4, 4] = float("inf")
+    a[25, 6, 2] = -float("inf")
+    z, w, info = eg.eigen_batch(a.clone())
+    zq, wq, iq = eg.eigen_batch(a.clone(), solver=eg.IMTQL2 | extra, path=path)
+    torch.cuda.synchronize()
+    assert torch.equal(info, iq)
+    assert bool(torch.isnan(w[bad]).any(1).all()) and bool(torch.isnan(wq[bad]).any(1).all())
+    ok = [k for k in range(L) if k not in bad]
+    assert bool(torch.isfinite(w[ok]).all()) and bool(torch.isfinite(z[ok]).all())
+    if n <= 64:
+        assert torch.equal(torch.isnan(z[bad]), torch.isnan(zq[bad]))
+    if int(info[1]) != 0:
+        assert torch.equal(z[bad].nan_to_num(), a[bad].nan_to_num())
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [9, 20, 33, 48, 64])
+def test_ql_split_kernels_in_large_batches(n, dtype):
+    """The separate QL kernels on batches that divide and conquer takes otherwise: with d
+    and e in LDS, and in registers (TQL2, and the order of the iteration); the bounds are
+    the reference checker's."""
+    L = 2100
+    print(f"[ql split] n={n} {np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(n)
+    b = rng.uniform(-1, 1, (L, n, n))
+    a = torch.from_numpy(((b + b.transpose(0, 2, 1)) / 2).astype(dtype)).to(DEV)
+    we = np.linalg.eigvalsh(a.cpu().numpy().astype(np.float64))
+    eps = float(np.finfo(dtype).eps)
+    tol = eps * (1023 if dtype == np.float64 else 31) * np.sqrt(n + 16.0) * np.abs(we).max(axis=1, keepdims=True)
+    for kw in (dict(path="split-lds"), dict(path="split", solver=eg.TQL2), dict(path="split", unsorted=True)):
+        z, w, info = eg.eigen_batch(a.clone(), **kw)
+        assert int(info.abs().max()) == 0
+        assert int(eg.check(a, w, z)[:, 3].max()) == 0
+        assert (np.abs(np.sort(w.cpu().numpy().astype(np.float64), axis=1) - we) <= tol).all()
