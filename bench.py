@@ -152,10 +152,10 @@ def time_phases(a0, steps, warmup, path="split"):
     """Per-phase HIP-event times (ms) of a path in separate kernels: the phases are
     issued as separate library calls on one stream with events between them.  For
     batches that take divide and conquer (from 2048 matrices) with n <= 64: tri =
-    eig_tri_wave_kernel (eig_tri_kernel for n <= 32), ql = nothing, apply =
-    eig_dc_kernel; larger n: tri = eig_tri_reg_kernel (n <= 256) or
-    eig_tri_stream_kernel, ql = the merges, apply = the back-transformation.
-    Returns {phase: mean ms}."""
+    eig_tri_wave_kernel (eig_tri_kernel for n <= 32), ql+apply = eig_dc_kernel (alone,
+    ql runs its merges for the eigenvalues, and apply runs them again); larger n: tri =
+    eig_tri_reg_kernel (n <= 256) or eig_tri_stream_kernel, ql = the merges, apply = the
+    back-transformation.  Returns {phase: mean ms}."""
     import numpy as np
     import torch
     import eigeng_batched as eg
@@ -166,14 +166,14 @@ def time_phases(a0, steps, warmup, path="split"):
                      device="cuda")
     info = torch.empty(L, dtype=torch.int32, device="cuda")
     stream = torch.cuda.current_stream()
-    names = ["tri", "ql", "apply"]
+    names = ["tri", "ql+apply"] if n <= 64 else ["tri", "ql", "apply"]
     rec = {p: [] for p in names}
     for i in range(warmup + steps):
         a.copy_(a0)
-        ev = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(len(names) + 1)]
         ev[0].record(stream)
         for j, p in enumerate(names):
-            eg.eigen_batch(a, w=w, info=info, workspace=ws, stream=stream, path=path, phases=[p])
+            eg.eigen_batch(a, w=w, info=info, workspace=ws, stream=stream, path=path, phases=p.split("+"))
             ev[j + 1].record(stream)
         torch.cuda.synchronize()
         if i >= warmup:

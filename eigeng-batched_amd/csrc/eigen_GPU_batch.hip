@@ -422,8 +422,8 @@ hipError_t launch_split(int L, int nm, int n, T *a, T *w, int *info, int solver,
 }
 
 // Divide and conquer path for n <= 64 on one chunk: q, de (ld rows apart) as in
-// DcLayout.  Phases: tridiagonalisation with Q; the second one nothing; merges and
-// store.  nanfail, only: see eig_dc_kernel.
+// DcLayout.  Phases: tridiagonalisation with Q; merges for eigenvalues and status alone
+// (no eigenvector column is stored); merges and store.  nanfail, only: see eig_dc_kernel.
 template <typename T, int NB, int NBT, int NLR>
 void launch_dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int ph, int kop, int nanfail, T *q, T *de,
                      int ld, const int *only, hipStream_t s)
@@ -444,7 +444,8 @@ void launch_dc_chunk(int L, int cur, int nm, int n, T *a, T *w, int *info, int p
                          q, de, ld, UvSplitArgs{}, only);
     }
   }
-  if (ph & FLAG_PH_APPLY)
+  if (!(ph & FLAG_PH_APPLY)) kop = kopt_no_vectors(kop, n);
+  if (ph & (FLAG_PH_QL | FLAG_PH_APPLY))
     hipLaunchKernelGGL((eig_dc_kernel<T, NB, NLR, false>), dim3((unsigned)cur), dim3(NB * NLR), 0, s, cur, nm, n, a,
                        (const T *)q, (const T *)de, ld, w, info, kop, nanfail, 1, (T *)nullptr, (T *)nullptr, 0, only);
 }

@@ -195,7 +195,8 @@ def eigen_batch(a, w=None, m: int | None = None, solver: int = IMTQL2, info=None
     tridiagonalisation on the full matrix instead of its lower triangle) or
     "split-ws" (split with the workspace-resident lower-triangle
     tridiagonalisation instead of the register-resident one).
-    phases (split path only): iterable of "tri", "ql", "apply" to run.
+    phases (paths in separate kernels): iterable of "tri", "ql", "apply" to run;
+    w and info are set by "ql", a by "apply".
     m < n: all n eigenvalues, eigenvectors of the first m only (columns m..n-1
     of each matrix are left unspecified).  unsorted: the QL / Jacobi order.
     """

@@ -101,7 +101,8 @@ enum eigen_GPU_batch_solver {
  *          that they fail (a host-forced test of its status);
  *   0x1000 / 0x2000 / 0x4000  run only the tridiagonalisation / QL (or merges) /
  *          apply phase of a path in separate kernels (L <= 16384): successive calls on one stream with
- *          one workspace compose the full solve, so each phase can be timed;
+ *          one workspace compose the full solve, so each phase can be timed; w and
+ *          info are set after the second phase, a after the third;
  *   0x8000 FP32 64 < n <= 128: the register split path (two-wave
  *          tridiagonalisation, lane-per-matrix QL, 64-row-block apply), TQL2's
  *          default there from 2048 matrices; 0x200 selects the large-order

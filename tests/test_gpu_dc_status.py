@@ -54,6 +54,28 @@ def test_large_fp32_chunk_and_its_phases():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,L", [(8, 2100), (16, 2100), (20, 2100), (32, 3000), (48, 2100), (64, 2100), (100, 2100)])
+def test_eigenvalues_after_the_second_phase(n, L, dtype):
+    """The first two phases, together or one by one: eigenvalues and status, as after the
+    QL recurrence, with a as it was; the third then stores the vectors."""
+    print(f"[phases] n={n} L={L} {dtype}", flush=True)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(n)
+    b = torch.rand((L, n, n), generator=g, device=DEV, dtype=dtype) - 0.5
+    a = (b + b.transpose(1, 2)).contiguous()
+    z, w, _ = eg.eigen_batch(a.clone())
+    ws = torch.empty(eg.bufsize(L, n, n, n, a.element_size()), dtype=torch.uint8, device=DEV)
+    for phases in ([["tri", "ql"], ["apply"]], [["tri"], ["ql"], ["apply"]], [["tri"], ["ql", "apply"]]):
+        zp, wp = a.clone(), torch.full_like(w, float("nan"))
+        info = torch.full((L,), -7, dtype=torch.int32, device=DEV)
+        for ph in phases:
+            if ph == ["apply"]:
+                assert torch.equal(wp, w) and torch.equal(zp, a) and int(info.abs().max()) == 0
+            eg.eigen_batch(zp, w=wp, info=info, workspace=ws, phases=ph)
+        assert torch.equal(wp, w) and torch.equal(zp, z) and int(info.abs().max()) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("n,L", [(8, 40), (16, 3000), (20, 40), (20, 600), (40, 40), (64, 2100), (65, 40), (100, 2100),
                                  (200, 40), (300, 8), (512, 4)])
 def test_merges_that_fail_are_reported(n, L, dtype):
