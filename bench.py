@@ -921,6 +921,9 @@ def main():
     flops = (10.0 / 3.0) * n ** 3
     bytes_alg = s * (n * (n + 1) / 2 + n * n + n)
     peak_c = PEAK_FP32_TFLOPS if args.dtype == "fp32" else PEAK_FP64_TFLOPS
+    tri_solver = "divide and conquer" if phases else "the tridiagonal eigenproblem"
+    steps_of = [f"Householder + {tri_solver} + back-transform", "Householder + TQL2 + back-transform",
+                "Jacobi"][args.solver]
     if phases:
         # the step is a sequence of kernels: the roof is taken over their summed
         # event-timed durations
@@ -950,7 +953,7 @@ def main():
         "vs_baseline": None,
         "dtype": "f32" if args.dtype == "fp32" else "f64",
         "data": "synthetic (seeded GPU generator, LETKF ensemble-space matrices)",
-        "config": {"workload": f"plain solver (Householder + IMTQL2 + back-transform), L={L} "
+        "config": {"workload": f"plain solver ({steps_of}), L={L} "
                                f"LETKF matrices n=nm=m={n} {args.dtype}, k={k_mem} p={p_obs} "
                                f"rho={rho} sigma={sigma}",
                    "L": L, "n": n, "solver": ["imtql2", "tql2", "jacobi"][args.solver]},

@@ -1,5 +1,5 @@
-// eig_tri_wave.hpp - Householder tridiagonalisation with Q for 32 < n <= 64, one
-// matrix per wave and no barrier: lane i holds row i of the full symmetric matrix
+// eig_tri_wave.hpp - Householder tridiagonalisation with Q for 32 < n <= 64, and for
+// 16 < n <= 32 in batches of up to 2048 matrices, one matrix per wave and no barrier: lane i holds row i of the full symmetric matrix
 // in strips of 16 registers, so every product with it is lane-local and the column
 // operands come from the lanes of the row inside the FMA (bcast_dot16, bcast_axpy16).
 // The convention is that of the other tridiagonalisations (eig_tri_reg.hpp).

@@ -47,8 +47,9 @@ __host__ __device__ constexpr int kopt_solver(int o) { return o & 0xff; }
 __host__ __device__ constexpr bool kopt_unsorted(int o) { return ((o >> 8) & 1) != 0; }
 constexpr int KOPT_CUT = 0x200;
 __host__ __device__ constexpr bool kopt_cut(int o) { return (o & KOPT_CUT) != 0; }
+// no eigenvector column written
 __host__ __device__ constexpr int kopt_no_vectors(int o, int n) { return (o & ~(0x3ff << 12)) | (n << 12); }
-__host__ __device__ constexpr int kopt_mdrop(int o) { return (o >> 12) & 0x3ff; }   // split path: rotation log full, solve with the fused kernel
+__host__ __device__ constexpr int kopt_mdrop(int o) { return (o >> 12) & 0x3ff; }
 
 // Offset of packed Householder column c (1 <= c) when column c' holds
 // roundup8(c') entries: sum_{c'=1}^{c-1} 8*ceil(c'/8).

@@ -230,10 +230,9 @@ bool use_dc(int L, int n, int tbytes, int solver)
 
 // 64 < n <= 512, the same interface: reflectors and a blocked back-transformation.
 // (FP32 n = 128, 8192 matrices: the two-wave tridiagonalisation that forms Q and a
-// product with it take 3.95 + 0.72 ms, reflectors 2.06 + 1.14.)
-bool use_dc_large(int L, int n, int tbytes, int solver)
+// product with it take 3.95 + 0.72 ms, reflectors 2.13 + 0.92.)
+bool use_dc_large(int L, int n, int solver)
 {
-  (void)tbytes;
   if (!dc_bits(solver) || n <= 64 || n > GL_NMAX) return false;
   return (solver & FLAG_DC) || !(solver & FLAG_SPLIT) || L >= SPLIT_MIN_L;
 }
@@ -345,7 +344,7 @@ size_t workspace_bytes(int L, int nm, int n, int m, int tbytes, int solver)
     const size_t own = WS_HEAD + DcLayout(L < lchunk(solver) ? L : lchunk(solver), n, tbytes).total;
     return own > other ? own : other;
   }
-  if (use_dc_large(L, n, tbytes, solver)) {
+  if (use_dc_large(L, n, solver)) {
     const size_t other = workspace_bytes(L, nm, n, m, tbytes, (solver & ~FLAG_DC) | FLAG_ROUTE_QL);
     const int ch = dc_large_chunk(n, tbytes, solver);
     const size_t own = WS_HEAD + DcLargeLayout(L < ch ? L : ch, n, tbytes).total;
@@ -1089,6 +1088,10 @@ hipError_t run_dc_large(int L, int nm, int n, T *a, T *w, int *info, int solver,
       const long long blocks = (long long)cur * nb16;
       hipLaunchKernelGGL((eig_dc_wyt_kernel<T>), dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, s, blocks, n,
                          nb16, (const T *)Wm, (const T *)bw, U);
+      // waves per SIMD: the most that keep V in registers (NT = 24 in FP64: 29 registers spill).
+      // One fewer / these / one more, us, 2048 matrices of n = 256 FP64 2665 / 2061 / 3281; 512
+      // of n = 384 FP32 844 / 841 / 1111, FP64 1902 / 1780 / 3760; 512 of n = 512 FP32
+      // 2527 / 1866 / 2967, FP64 - / 4136 / 7722; n = 128, and FP32 n = 256, all three alike.
       constexpr int W8 = tb == 8 ? 3 : 4, W16 = tb == 8 ? 2 : 3, W24 = tb == 8 ? 2 : 3, W32 = tb == 8 ? 1 : 2;
       if (n <= 128) launch_dc_back<T, 8, W8>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
       else if (n <= 256) launch_dc_back<T, 16, W16>(cur, n, nm, mcols, Wm, U, Z[0], ac, st, s);
@@ -1115,7 +1118,7 @@ hipError_t run(int L, int nm, int n, int m, T *a, T *w, void *wk, hipStream_t s,
   // kernel options: solver, order of the output, eigenvector columns not stored
   int kop = kopt_make(base, (solver & FLAG_UNSORTED) != 0, n - m);
   const int tb = (int)sizeof(T);
-  const bool dc = use_dc(L, n, tb, solver), dcl = use_dc_large(L, n, tb, solver);
+  const bool dc = use_dc(L, n, tb, solver), dcl = use_dc_large(L, n, solver);
   // phases: of a batch whose QL path is one in separate kernels, or asked for with FLAG_DC
   if ((solver & FLAG_PH_ALL) && !((dc || dcl) && (solver & FLAG_DC)) && !use_split(L, n, tb, solver) &&
       !use_split_large(L, n, tb, solver) && !use_split128(L, n, tb, solver))
