@@ -43,6 +43,7 @@
 // and 3.2, FP32 2.1 ms; 64 matrices of n = 200 in FP64 0.62 and 0.44 ms.
 #pragma once
 #include "common.hpp"
+#include "eig_tri_again.hpp"
 
 namespace eigmi {
 
@@ -260,6 +261,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
   const TriSlots<NB, NW> sl(wv);
   T *__restrict__ xw = S.xw[wv];
   T A[KT][16];
+  bool again = false;
 
   for (long long mat = blockIdx.x; mat < L; mat += gridDim.x) {
     // n and nm re-read opaquely per matrix: otherwise the per-element load
@@ -400,12 +402,28 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
       if (fresh) tr_publish<T, NB, NW>(r2, A, sl, lane, S);
     }
     __syncthreads();
+    again = again || tri_lost(S.beta, n);
     for (int i = tid; i < nv; i += NT) {
       de[(size_t)i * ld + mat] = S.d[i];
       de[(size_t)(nv + i) * ld + mat] = S.e[i];
       bws[(size_t)mat * nv + i] = S.beta[i];
     }
     __syncthreads();
+  }
+  if (__builtin_expect(again, 0)) {
+    // of this workgroup's matrices those that are lost (few, and none as a rule)
+    for (long long mat = blockIdx.x; mat < L; mat += gridDim.x) {
+      __syncthreads();                                      // every read of S is done
+      for (int i = tid; i < n; i += NT) S.beta[i] = bws[(size_t)mat * n + i];
+      __syncthreads();
+      if (!tri_lost(S.beta, n)) continue;
+      tri_again<T, NT>(mat, n, nm, a, W, S.u, S.p, S.d, S.e, S.beta, S.pcol);
+      for (int i = tid; i < n; i += NT) {
+        de[(size_t)i * ld + mat] = S.d[i];
+        de[(size_t)(n + i) * ld + mat] = S.e[i];
+        bws[(size_t)mat * n + i] = S.beta[i];
+      }
+    }
   }
 }
 
