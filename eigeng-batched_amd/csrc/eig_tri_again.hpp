@@ -38,9 +38,10 @@ __device__ __forceinline__ bool tri_lost(const T *__restrict__ beta, int n)
 
 // Matrix mat of the batch a; its slot of Ws.  The convention of the callers: u_c in
 // W(0:c-1, c), d, e, beta of n entries; u, p: n entries, red: one for every wave, all in LDS.
-// All NT threads of the workgroup call it.
+// All NT threads of the workgroup call it.  False, and nothing changed, for a matrix that is
+// not finite.
 template <typename T, int NT>
-__device__ __forceinline__ void tri_again(long long mat, int n, int nm, const T *__restrict__ a, T *Ws, T *u, T *p,
+__device__ __forceinline__ bool tri_again(long long mat, int n, int nm, const T *__restrict__ a, T *Ws, T *u, T *p,
                                           T *d, T *e, T *beta, T *red)
 {
   // opaque: nothing of this is computed, and held in registers, before the caller's columns
@@ -62,13 +63,13 @@ __device__ __forceinline__ void tri_again(long long mat, int n, int nm, const T 
   __syncthreads();                                          // the caller's stores to W are done
   T mx = T(0);                                              // the matrix's largest entry
   auto up = [&](T x) { mx = x > mx ? x : mx; };
+  const T inf = std::numeric_limits<T>::infinity();
 #pragma unroll 1
   for (int j = tid >> 6; j < n; j += NT / 64)
 #pragma unroll 1
-    for (int i = tid & 63; i < n; i += 64) {
-      const T x = Ain[(i < j ? i : j) + (size_t)(i < j ? j : i) * nm];
-      W[i + (size_t)j * n] = x;
-      up(abs_(x));
+    for (int i = tid & 63; i <= j; i += 64) {
+      const T x = abs_(Ain[i + (size_t)j * nm]);
+      up(x < inf ? x : inf);
     }
   up(lane_move(mx, MvX1()));
   up(lane_move(mx, MvX2()));
@@ -78,6 +79,13 @@ __device__ __forceinline__ void tri_again(long long mat, int n, int nm, const T 
   up(lane_move(mx, MvX32()));
   share(mx);
   for (int q = 0; q < NT / 64; ++q) up(red[q]);
+  if (!(mx < inf)) return false;
+#pragma unroll 1
+  for (int j = tid >> 6; j < n; j += NT / 64)
+#pragma unroll 1
+    for (int i = tid & 63; i < n; i += 64)
+      W[i + (size_t)j * n] = Ain[(i < j ? i : j) + (size_t)(i < j ? j : i) * nm];
+  __syncthreads();
 #pragma unroll 1
   for (int c = n - 1; c >= 1; --c) {
     T *col = W + (size_t)c * n;
@@ -103,7 +111,7 @@ __device__ __forceinline__ void tri_again(long long mat, int n, int nm, const T 
     T t = T(0);
     for (int i = tid; i < c; i += NT) {
       T y = T(0);
-#pragma unroll 1
+#pragma unroll 8
       for (int j = 0; j < c; ++j) y = fma_(W[i + (size_t)j * n], u[j], y);
       y *= b;
       p[i] = y;
@@ -126,6 +134,7 @@ __device__ __forceinline__ void tri_again(long long mat, int n, int nm, const T 
     e[n - 1] = beta[0] = T(0);
   }
   __syncthreads();
+  return true;
 }
 
 } // namespace eigmi

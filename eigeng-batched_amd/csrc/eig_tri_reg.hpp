@@ -416,8 +416,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
       __syncthreads();                                      // every read of S is done
       for (int i = tid; i < n; i += NT) S.beta[i] = bws[(size_t)mat * n + i];
       __syncthreads();
-      if (!tri_lost(S.beta, n)) continue;
-      tri_again<T, NT>(mat, n, nm, a, W, S.u, S.p, S.d, S.e, S.beta, S.pcol);
+      if (!tri_lost(S.beta, n) || !tri_again<T, NT>(mat, n, nm, a, W, S.u, S.p, S.d, S.e, S.beta, S.pcol)) continue;
       for (int i = tid; i < n; i += NT) {
         de[(size_t)i * ld + mat] = S.d[i];
         de[(size_t)(n + i) * ld + mat] = S.e[i];

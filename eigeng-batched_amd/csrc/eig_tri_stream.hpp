@@ -304,7 +304,7 @@ __global__ __launch_bounds__(TS_NT) void eig_tri_stream_kernel(int L, int nm, in
     }
     __syncthreads();
     if (__builtin_expect(tri_lost(S.beta, n), 0))
-      tri_again<T, TS_NT>(mat, n, nm, a, W, S.U[0], S.V[0], S.d, S.e, S.beta, S.dot);
+      (void)tri_again<T, TS_NT>(mat, n, nm, a, W, S.U[0], S.V[0], S.d, S.e, S.beta, S.dot);
     for (int i = tid; i < n; i += TS_NT) {
       de[(size_t)i * ld + mat] = S.d[i];
       de[(size_t)(n + i) * ld + mat] = S.e[i];

@@ -136,10 +136,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   }
   if (__builtin_expect(__ballot(tri_lost(bv)) != 0ull, 0)) {
     T *l = &S.G[0][0];
-    tri_again<T, 64>(mat, n, nm, a, qws, S.x, S.p, l, l + 64, l + 128, l + 192);
-    dv = lane < n ? l[lane] : T(0);
-    ev = lane < n ? l[64 + lane] : T(0);
-    bv = lane < n ? l[128 + lane] : T(0);
+    if (tri_again<T, 64>(mat, n, nm, a, qws, S.x, S.p, l, l + 64, l + 128, l + 192)) {
+      dv = lane < n ? l[lane] : T(0);
+      ev = lane < n ? l[64 + lane] : T(0);
+      bv = lane < n ? l[128 + lane] : T(0);
+    }
   }
   if (lane < n) {
     de[(size_t)lane * ld + mat] = dv;
