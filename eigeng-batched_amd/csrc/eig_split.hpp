@@ -99,19 +99,40 @@ __global__ __launch_bounds__(64 * GroupShape<NB>::NW) void eig_tri_kernel(int L,
     Q = qws + (size_t)mat * (size_t)n * (size_t)n;
   }
   WaveLds<T, NB> &S = smem[g];
-  T R[NB], dv[NW], ev[NW];
-  wave_front<T, NB>(A, nm, n, k, kl, wv, S, R, dv, ev);
+  bool lost = false;
+  {
+    T R[NB], dv[NW], ev[NW], bv[NW];
+    wave_front<T, NB>(A, nm, n, k, kl, wv, S, R, dv, ev, bv);
 #pragma unroll
-  for (int j = 0; j < NB; ++j)
-    if (j < n && k < n) Q[k + (size_t)j * n] = R[j];
-  if (wv == 0) {
-    // d and e are lane-distributed (entry kl + NL h in dv[h]) and the same in every wave
+    for (int j = 0; j < NB; ++j)
+      if (j < n && k < n) Q[k + (size_t)j * n] = R[j];
+    if (wv == 0) {
+      // d and e are lane-distributed (entry kl + NL h in dv[h]) and the same in every wave
 #pragma unroll
-    for (int h = 0; h < NW; ++h) {
-      const int i = kl + NL * h;
-      if (i < n) {
-        de[(size_t)i * ld + mat] = dv[h];
-        de[(size_t)(eoff + i) * ld + mat] = ev[h];
+      for (int h = 0; h < NW; ++h) {
+        const int i = kl + NL * h;
+        if (i < n) {
+          de[(size_t)i * ld + mat] = dv[h];
+          de[(size_t)(eoff + i) * ld + mat] = ev[h];
+        }
+      }
+    }
+    lost = tri_lost(bv[0]);
+  }
+  // the orders that divide and conquer takes from here
+  if constexpr (NB <= 32 && !LIST) {
+    if (__builtin_expect(group_ballot<NB>(lost) != 0ull, 0)) {
+      // opaque: no address of this is held in registers while the first reduction runs
+      int i = kl, nn = n, ldm = nm;
+      asm volatile("" : "+v"(i), "+s"(nn), "+s"(ldm));
+      T R[NB], dv[1], ev[1], bv[1];
+      wave_front<T, NB, true>(A, ldm, nn, i, i, 0, S, R, dv, ev, bv);
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        if (j < nn && i < nn) Q[i + (size_t)j * nn] = R[j];
+      if (i < nn) {
+        de[(size_t)i * ld + mat] = dv[0];
+        de[(size_t)(nn + i) * ld + mat] = ev[0];
       }
     }
   }

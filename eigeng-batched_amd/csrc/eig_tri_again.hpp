@@ -6,8 +6,8 @@
 // (FP64) after a few columns, sums of squares there are subnormal or zero and 1 / (ul anorm)
 // overflows.  The reductions of eig_tri_wave.hpp, eig_tri_reg.hpp and eig_tri_stream.hpp
 // find that out from beta after their last column (a test in every column costs FP64
-// n = 32, L = 1024 3 us of 84), and the workgroup starts again here: the unblocked form in
-// place in W, which sets a column to zero if its norm is below eps times the matrix's
+// n = 32, L = 1024 3 us of 84), and the workgroup starts again here (eig_tri_kernel for
+// n <= 32 in its own form): the unblocked form in place in W, which sets a column to zero if its norm is below eps times the matrix's
 // largest entry, a backward error of eps.  A matrix that is itself as small as that comes to
 // the same end as before.
 #pragma once

@@ -27,6 +27,7 @@
 // QL rotations are accumulated into it, which gives the same product Q * Z_QL.
 #pragma once
 #include "common.hpp"
+#include "eig_tri_again.hpp"
 
 namespace eigmi {
 
@@ -180,15 +181,19 @@ __device__ __forceinline__ void apply_two_sweeps(T (&Zr)[NB], const typename vec
 
 // Front half shared by the fused and the split solvers: load row k of matrix A
 // (upper triangle only), Householder tridiagonalisation, Q = H_{n-1}...H_1 in R.
-// On return R holds row k of Q and dv / ev the lane-distributed diagonal and
-// off-diagonal (replicated in every wave of the group).
-template <typename T, int NB>
+// On return R holds row k of Q and dv / ev / bv the lane-distributed diagonal,
+// off-diagonal and reflector scales (replicated in every wave of the group).
+// AGAIN: a column below eps of the matrix's largest entry is set to zero where its
+// squares underflow (eig_tri_again.hpp; one wave per matrix).
+template <typename T, int NB, bool AGAIN = false>
 __device__ __forceinline__ void wave_front(const T *__restrict__ A, int nm, int n, int k, int kl, int wv,
                                            WaveLds<T, NB> &S, T (&R)[NB],
-                                           T (&dv)[GroupShape<NB>::NW], T (&ev)[GroupShape<NB>::NW])
+                                           T (&dv)[GroupShape<NB>::NW], T (&ev)[GroupShape<NB>::NW],
+                                           T (&bv)[GroupShape<NB>::NW])
 {
   constexpr int NL = GroupShape<NB>::NL, NW = GroupShape<NB>::NW;
   constexpr int NBLK = NB / 8;
+  static_assert(!AGAIN || NW == 1, "");
   // R holds row k of A during the reduction and row k of Q afterwards.
   // ---- load: row k of the symmetric matrix from the upper triangle ----------
   // Columns j > k come from row k of the upper triangle (coalesced across
@@ -221,7 +226,12 @@ __device__ __forceinline__ void wave_front(const T *__restrict__ A, int nm, int 
     }
   }
 
-  T bv[NW];
+  T mx = T(0);
+  if constexpr (AGAIN) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) mx = abs_(R[j]) > mx ? abs_(R[j]) : mx;
+    mx = group_reduce<NL>(mx, [](T x, T y) { return x > y ? x : y; });
+  }
 #pragma unroll
   for (int h = 0; h < NW; ++h) { dv[h] = T(0); ev[h] = T(0); bv[h] = T(0); }
 
@@ -236,8 +246,10 @@ __device__ __forceinline__ void wave_front(const T *__restrict__ A, int nm, int 
     gsync<NW>();
     T uk = (k < c) ? S.rowbuf[k] : T(0);
     const T dc = S.rowbuf[c];
-    const T ulast = S.rowbuf[c - 1];
-    const T sig = gsum<NB>(uk * uk, S.red, 0, wv, kl);
+    T ulast = S.rowbuf[c - 1];
+    T sig = gsum<NB>(uk * uk, S.red, 0, wv, kl);
+    if constexpr (AGAIN)
+      if (sig < TriTiny<T>::SUM && sqrt_(sig) <= eps_of<T>() * mx) uk = ulast = sig = T(0);
     const T anorm = -sign_(sqrt_(sig), ulast);
     const T ul = ulast - anorm;
     const T beta = T(1) / nz(ul * anorm);
@@ -334,7 +346,10 @@ __device__ __forceinline__ void wave_solve(T *__restrict__ A, int nm, int n, T *
   constexpr int NL = GroupShape<NB>::NL, NW = GroupShape<NB>::NW;
   typedef typename vec2<T>::type T2;
   T R[NB], dv[NW], ev[NW];
-  wave_front<T, NB>(A, nm, n, k, kl, wv, S, R, dv, ev);
+  {
+    T bv[NW];
+    wave_front<T, NB>(A, nm, n, k, kl, wv, S, R, dv, ev, bv);
+  }
 
   // ---- QL with eigenvectors accumulated into Z = R --------------------------
   // Everything below is per wave (replicated vectors, a private (c, s) array):
