@@ -80,6 +80,7 @@ __global__ __launch_bounds__(TS_NT) void eig_tri_stream_kernel(int L, int nm, in
   __shared__ TriStreamLds<T, NBP, TS_NW> S;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  bool again = false;
   for (long long mat = blockIdx.x; mat < L; mat += gridDim.x) {
     const T *__restrict__ A = a + (size_t)mat * (size_t)nm * (size_t)n;
     T *__restrict__ Wm = W + (size_t)mat * n * n;
@@ -303,14 +304,29 @@ __global__ __launch_bounds__(TS_NT) void eig_tri_stream_kernel(int L, int nm, in
       S.d[0] = x;
     }
     __syncthreads();
-    if (__builtin_expect(tri_lost(S.beta, n), 0))
-      (void)tri_again<T, TS_NT>(mat, n, nm, a, W, S.U[0], S.V[0], S.d, S.e, S.beta, S.dot);
+    again = again || tri_lost(S.beta, n);
     for (int i = tid; i < n; i += TS_NT) {
       de[(size_t)i * ld + mat] = S.d[i];
       de[(size_t)(n + i) * ld + mat] = S.e[i];
       bws[(size_t)mat * n + i] = S.beta[i];
     }
     __syncthreads();
+  }
+  if (__builtin_expect(again, 0)) {
+    // as in eig_tri_reg_kernel
+    for (long long mat = blockIdx.x; mat < L; mat += gridDim.x) {
+      __syncthreads();
+      for (int i = tid; i < n; i += TS_NT) S.beta[i] = bws[(size_t)mat * n + i];
+      __syncthreads();
+      if (!tri_lost(S.beta, n) ||
+          !tri_again<T, TS_NT>(mat, n, nm, a, W, S.U[0], S.V[0], S.d, S.e, S.beta, S.dot))
+        continue;
+      for (int i = tid; i < n; i += TS_NT) {
+        de[(size_t)i * ld + mat] = S.d[i];
+        de[(size_t)(n + i) * ld + mat] = S.e[i];
+        bws[(size_t)mat * n + i] = S.beta[i];
+      }
+    }
   }
 }
 
